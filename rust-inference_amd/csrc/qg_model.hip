@@ -821,17 +821,29 @@ int mfail(qg_model *m, int st, const char *what, hipError_t e = hipSuccess)
         if (e_ != hipSuccess) return mfail((m), QG_ERR_HIP, #call, e_);       \
     } while (0)
 
+// n zeroed elements (zeroed in stream order: every user of them is on the
+// context's stream)
 template <class T> int dalloc(qg_model *m, T **p, size_t n)
 {
     void *d = nullptr;
     hipError_t e = hipMalloc(&d, (n ? n : 1) * sizeof(T));
     if (e != hipSuccess) return mfail(m, QG_ERR_OUT_OF_MEMORY, "hipMalloc", e);
-    e = hipMemset(d, 0, (n ? n : 1) * sizeof(T));
-    if (e != hipSuccess) { (void)hipFree(d); return mfail(m, QG_ERR_HIP, "hipMemset", e); }
+    e = hipMemsetAsync(d, 0, (n ? n : 1) * sizeof(T), m->ctx->stream);
+    if (e != hipSuccess) { (void)hipFree(d); return mfail(m, QG_ERR_HIP, "hipMemsetAsync", e); }
     m->allocs.push_back(d);
     m->alloc_bytes += (n ? n : 1) * sizeof(T);
     *p = (T *)d;
     return QG_OK;
+}
+
+// hipMemcpy in the order of the context's stream, and waited for.  The legacy
+// stream (hipMemcpy, hipMemset) stays unused: its operations fail while any
+// thread of the process captures a graph, and break that capture.
+hipError_t copy_wait(qg_model *m, void *dst, const void *src, size_t n, hipMemcpyKind kind)
+{
+    const hipError_t e = hipMemcpyAsync(dst, src, n, kind, m->ctx->stream);
+    const hipError_t es = hipStreamSynchronize(m->ctx->stream);
+    return e != hipSuccess ? e : es;
 }
 
 void drop_graphs(qg_model *m)
@@ -1552,8 +1564,8 @@ int qg_model_create(qg_ctx *ctx, const qg_model_config *cfg, qg_model **out)
             st[pos * half + i] = sinf(angle);
         }
     if ((rc = dalloc(m, &m->cos_t, np)) || (rc = dalloc(m, &m->sin_t, np))) { free_model(m); return rc; }
-    if ((e = hipMemcpy(m->cos_t, ct.data(), np * sizeof(float), hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(m->sin_t, st.data(), np * sizeof(float), hipMemcpyHostToDevice)) != hipSuccess ||
+    if ((e = copy_wait(m, m->cos_t, ct.data(), np * sizeof(float), hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = copy_wait(m, m->sin_t, st.data(), np * sizeof(float), hipMemcpyHostToDevice)) != hipSuccess ||
         (e = hipHostMalloc((void **)&m->h_recent, qgm::kRecentMax * sizeof(uint32_t), hipHostMallocDefault)) !=
             hipSuccess ||
         (e = hipHostMalloc((void **)&m->h_token, sizeof(uint32_t), hipHostMallocDefault)) != hipSuccess ||
@@ -1633,8 +1645,7 @@ int qg_model_set_vector(qg_model *m, uint32_t which, uint32_t layer, const float
     }
     if (n != want) return mfail(m, QG_ERR_SHAPE, "vector length does not match the config");
     QGM_HIP(m, hipSetDevice(m->ctx->device));
-    QGM_HIP(m, hipStreamSynchronize(m->ctx->stream));
-    QGM_HIP(m, hipMemcpy(dst, v, n * sizeof(float), hipMemcpyHostToDevice));
+    QGM_HIP(m, copy_wait(m, dst, v, n * sizeof(float), hipMemcpyHostToDevice));
     return QG_OK;
 }
 
@@ -1777,7 +1788,7 @@ int qg_model_generate(qg_model *m, const uint32_t *prompt, size_t n_prompt, size
     QGM_HIP(m, hipStreamSynchronize(st));
     m->seq = 0;                                                     // fresh caches (model.rs:341-346)
     if (n_prompt == 0) return QG_OK;
-    QGM_HIP(m, hipMemcpy(m->d_hist, prompt, n_prompt * sizeof(uint32_t), hipMemcpyHostToDevice));
+    QGM_HIP(m, copy_wait(m, m->d_hist, prompt, n_prompt * sizeof(uint32_t), hipMemcpyHostToDevice));
     // model.rs:370-374 passes the last 64 tokens; the sampler keeps `window` of them
     const uint32_t win = window > qgm::kRecentMax ? qgm::kRecentMax : (uint32_t)window;
     int rc;
@@ -1805,7 +1816,7 @@ int qg_model_generate(qg_model *m, const uint32_t *prompt, size_t n_prompt, size
     auto t2 = clk::now();
     m->seq = n_prompt + n_new;
     if (n_new)
-        QGM_HIP(m, hipMemcpy(out_tokens, m->d_hist + n_prompt, n_new * sizeof(uint32_t), hipMemcpyDeviceToHost));
+        QGM_HIP(m, copy_wait(m, out_tokens, m->d_hist + n_prompt, n_new * sizeof(uint32_t), hipMemcpyDeviceToHost));
     if (prefill_s) *prefill_s = std::chrono::duration<double>(t1 - t0).count();
     if (decode_s) *decode_s = std::chrono::duration<double>(t2 - t1).count();
     return QG_OK;

@@ -546,8 +546,12 @@ int qg_upload(qg_ctx *ctx, const void *raw, size_t nbytes, uint32_t type, size_t
     uint8_t *d = nullptr;
     hipError_t e = qg_alloc_injected(ctx) ? hipErrorOutOfMemory : hipMalloc((void **)&d, need + qg::kTailPad);
     if (e != hipSuccess) return fail(ctx, QG_ERR_OUT_OF_MEMORY, "hipMalloc matrix", e);
-    e = hipMemcpy(d, raw, need, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(d + need, 0, qg::kTailPad);
+    // on the context's stream: the legacy stream's operations fail while any
+    // thread of the process captures a graph, and break that capture
+    e = hipMemcpyAsync(d, raw, need, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(d + need, 0, qg::kTailPad, ctx->stream);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = es;
     if (e != hipSuccess) {
         (void)hipFree(d);
         return fail(ctx, QG_ERR_HIP, "upload", e);

@@ -108,3 +108,49 @@ def test_models_in_parallel_threads(rinf, oracle, synth):
     for s in seeds:
         assert np.array_equal(got[s], alone[s]), (s, got[s][:8], alone[s][:8])
     assert not np.array_equal(alone[seeds[0]], alone[seeds[1]])
+
+
+def test_model_while_another_thread_captures(rinf, oracle, synth):
+    """A model is built and generates on one thread while another is in the
+    middle of capturing a graph of its own: neither touches the legacy stream,
+    so both end as they would alone."""
+    import torch
+    from test_decode_gpu import SMALL, build
+    prompt = (np.arange(5, 25, dtype=np.uint32) * 11) % SMALL["vocab_size"]
+
+    def run():
+        c = rinf.GpuContext(0)
+        try:
+            dev, _, _ = build(rinf, synth, oracle, c, dict(SMALL), "q4_k_m", 23, 64)
+            try:
+                return np.array(dev.generate(prompt, 8)[0])
+            finally:
+                dev.close()
+        finally:
+            c.close()
+
+    alone = run()
+    x = torch.ones(64, device="cuda")
+    y = torch.zeros(64, device="cuda")
+    got = []
+
+    def work():
+        try:
+            got.append(run())
+        except Exception as e:                         # reported by the main thread
+            got.append(e)
+
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, capture_error_mode="thread_local"):
+        y.add_(x)
+        th = threading.Thread(target=work)
+        th.start()
+        th.join(timeout=100)
+        y.add_(x)
+    assert not th.is_alive()
+    assert not isinstance(got[0], Exception), got[0]
+    assert np.array_equal(got[0], alone)
+    for i in range(1, 4):
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, 2.0 * i * x)
