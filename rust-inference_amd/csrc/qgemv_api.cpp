@@ -550,13 +550,21 @@ int qg_upload(qg_ctx *ctx, const void *raw, size_t nbytes, uint32_t type, size_t
     // thread of the process captures a graph, and break that capture
     e = hipMemcpyAsync(d, raw, need, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(d + need, 0, qg::kTailPad, ctx->stream);
-    const hipError_t es = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = es;
     if (e != hipSuccess) {
+        (void)hipStreamSynchronize(ctx->stream);
         (void)hipFree(d);
         return fail(ctx, QG_ERR_HIP, "upload", e);
     }
+    // (waits for the copy where it repacks)
     rc = new_mat(ctx, d, need, type, rows, cols, true, out);
+    if (rc != QG_OK || !(*out)->d_rp) {
+        e = hipStreamSynchronize(ctx->stream);
+        if (rc == QG_OK && e != hipSuccess) {
+            drop_mat(ctx, *out);                         // frees d
+            *out = nullptr;
+            return fail(ctx, QG_ERR_HIP, "upload", e);
+        }
+    }
     if (rc != QG_OK) (void)hipFree(d);
     return rc;
 }
