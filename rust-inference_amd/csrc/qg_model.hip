@@ -793,6 +793,13 @@ struct qg_model {
     // the QKV output's K splits: [Q; K; V] in one launch (one type), or
     // [Q; K] and V in two (V another type: its few row tiles take more slices)
     uint32_t pf_s_qkv1 = 1, pf_s_qk = 1, pf_s_v = 1;
+    // prefill of more than kPfMaxTokens tokens (qg_prefill_wide.hip), up to
+    // pf_wide tokens per chunk: the same buffers for whole tiles of tokens
+    uint32_t pf_wide = 0;
+    float *wd_h[2] = {nullptr, nullptr}, *wd_qkv = nullptr, *wd_ao = nullptr, *wd_ao2 = nullptr, *wd_g = nullptr,
+          *wd_fo = nullptr, *wd_scl = nullptr;
+    uint8_t *wd_xp = nullptr;
+    uint32_t *wd_rec = nullptr;
     // captured graphs per attention mode: [0] the split attention
     // (attn_rope_split_k + attn_combine_k), [1] whole heads in one workgroup
     // each (attn_rope_head_k), [2] two position ranges per head merged in the
@@ -1375,11 +1382,22 @@ int pf_planes(qg_model *m, const float *a, uint32_t na, const float *b, uint32_t
     return r ? mfail(m, QG_ERR_HIP, "prefill planes launch", hipGetLastError()) : QG_OK;
 }
 
+// The logits of token ntok - 1 from the residual stream h and the last
+// down GEMM's ns slices (transformer.rs:87-97): the final norm inside the
+// lm_head GEMV.
+int pf_logits(qg_model *m, const float *h, const float *fo, uint32_t ns, size_t sstride, uint32_t ntok)
+{
+    const size_t E = m->cfg.embed_dim, last = (size_t)(ntok - 1) * E;
+    if (qg::launch_pf_sum(fo + last, ns, sstride, E, m->pf_last, (ihipStream_t *)m->ctx->stream))
+        return mfail(m, QG_ERR_HIP, "prefill sum", hipGetLastError());
+    return gemv_norm(m, m->lm, h + last, m->pf_last, m->final_norm, nullptr, m->logits);
+}
+
 // Transformer::forward (transformer.rs:63-98) for tokens d_tok[0..ntok) (on
 // device) at positions / cache slots s0 .. s0 + ntok - 1, every layer's
-// projections as GEMMs over the chunk; leaves the last token's logits in
-// m->logits.
-int pf_chunk(qg_model *m, const uint32_t *d_tok, uint32_t ntok, uint32_t s0)
+// projections as GEMMs over the chunk; with `last`, leaves the last token's
+// logits in m->logits.
+int pf_chunk(qg_model *m, const uint32_t *d_tok, uint32_t ntok, uint32_t s0, bool last)
 {
     const qg_model_config &c = m->cfg;
     hipStream_t st = m->ctx->stream;
@@ -1443,10 +1461,138 @@ int pf_chunk(qg_model *m, const uint32_t *d_tok, uint32_t ntok, uint32_t s0)
             return rc;
     }
     // the last token's final norm of h + fo inside the lm_head GEMV (transformer.rs:87-97)
-    const size_t last = (size_t)(ntok - 1) * E;
-    if (qg::launch_pf_sum(m->pf_fo + last, m->pf_s_down, T * E, E, m->pf_last, sti))
-        return mfail(m, QG_ERR_HIP, "prefill sum", hipGetLastError());
-    return gemv_norm(m, m->lm, h + last, m->pf_last, m->final_norm, nullptr, m->logits);
+    return last ? pf_logits(m, h, m->pf_fo, m->pf_s_down, T * E, ntok) : QG_OK;
+}
+
+// Every layer matrix a repacked one that the wide GEMM takes, rows short
+// enough for its planes kernel.
+bool wide_supported(const qg_model *m)
+{
+    if (m->cfg.max_seq_len <= qg::kPfMaxTokens) return false;
+    for (int s = 0; s < kSlots; s++)
+        for (const qg_mat *p : m->w[s])
+            if (!qg::wide_mat_ok(pf_mat(p, nullptr), p->cols)) return false;
+    return true;
+}
+
+// K slices of the four GEMM groups for tt token tiles (V apart from Q and K:
+// its own)
+struct WideSplit {
+    uint32_t qkv, qk, v, o, gu, down;
+};
+WideSplit wide_splits(const qg_model *m, uint32_t tt)
+{
+    const size_t E = m->cfg.embed_dim, H = m->cfg.hidden_dim;
+    const uint32_t tq = qg::wide_tiles(m->q_dim), tk = qg::wide_tiles(m->kv_dim), te = qg::wide_tiles(E);
+    return WideSplit{qg::wide_split(tq + 2 * tk, tt, E), qg::wide_split(tq + tk, tt, E), qg::wide_split(tk, tt, E),
+                     qg::wide_split(te, tt, m->q_dim), qg::wide_split(2 * qg::wide_tiles(H), tt, E),
+                     qg::wide_split(te, tt, H)};
+}
+
+int wide_alloc(qg_model *m)
+{
+    if (m->pf_wide) return QG_OK;
+    const size_t E = m->cfg.embed_dim, H = m->cfg.hidden_dim, ldq = m->q_dim + 2 * (size_t)m->kv_dim;
+    const uint32_t cap = std::min<uint32_t>(qg::kWideMax, (m->cfg.max_seq_len + qg::kWideTile - 1) / qg::kWideTile * qg::kWideTile);
+    const size_t kmax = std::max({E, H, (size_t)m->q_dim}), T = cap;
+    // rows of the GEMM outputs: their slices at every number of token tiles
+    size_t rq = 0, ro = 0, rg = 0, rd = 0;
+    for (uint32_t tt = 1; tt <= cap / qg::kWideTile; tt++) {
+        const WideSplit s = wide_splits(m, tt);
+        const size_t t = (size_t)tt * qg::kWideTile;
+        rq = std::max(rq, t * std::max({s.qkv, s.qk, s.v}));
+        ro = std::max(ro, t * s.o);
+        rg = std::max(rg, t * s.gu);
+        rd = std::max(rd, t * s.down);
+    }
+    int rc;
+    if ((!m->wd_h[0] && (rc = dalloc(m, &m->wd_h[0], T * E))) || (!m->wd_h[1] && (rc = dalloc(m, &m->wd_h[1], T * E))) ||
+        (!m->wd_qkv && (rc = dalloc(m, &m->wd_qkv, rq * ldq))) || (!m->wd_ao && (rc = dalloc(m, &m->wd_ao, T * m->q_dim))) ||
+        (!m->wd_ao2 && (rc = dalloc(m, &m->wd_ao2, ro * E))) || (!m->wd_g && (rc = dalloc(m, &m->wd_g, rg * 2 * H))) ||
+        (!m->wd_fo && (rc = dalloc(m, &m->wd_fo, rd * E))) || (!m->wd_xp && (rc = dalloc(m, &m->wd_xp, T * kmax * 4))) ||
+        (!m->wd_rec && (rc = dalloc(m, &m->wd_rec, T * kmax / 32))) || (!m->wd_scl && (rc = dalloc(m, &m->wd_scl, T))))
+        return rc;
+    m->pf_wide = cap;
+    return QG_OK;
+}
+
+// n matrices over the same x, a launch per run of one type and row grouping
+int wide_gemm(qg_model *m, const qg::PfMat *mats, int n, size_t cols, uint32_t ntok, uint32_t ldy, uint32_t slices,
+              size_t sstride)
+{
+    for (int i = 0; i < n;) {
+        int k = i + 1;
+        while (k < n && mats[k].type == mats[i].type && (mats[k].g == 1) == (mats[i].g == 1)) k++;
+        if (qg::launch_wide_gemm(mats + i, k - i, cols, m->wd_xp, m->wd_rec, m->wd_scl, ntok, ldy, slices, sstride,
+                                 (ihipStream_t *)m->ctx->stream))
+            return mfail(m, QG_ERR_HIP, "prefill GEMM launch", hipGetLastError());
+        i = k;
+    }
+    return QG_OK;
+}
+
+int wide_planes(qg_model *m, const float *a, uint32_t na, const float *b, uint32_t nb, size_t sstride, float *sum_out,
+                const float *nw, size_t n, size_t lda, int mode, uint32_t ntok)
+{
+    if (qg::launch_wide_planes(a, na, b, nb, sstride, sum_out, nw, n, lda, mode, m->cfg.norm_eps, m->wd_xp, m->wd_rec,
+                               m->wd_scl, ntok, (ihipStream_t *)m->ctx->stream))
+        return mfail(m, QG_ERR_HIP, "prefill planes launch", hipGetLastError());
+    return QG_OK;
+}
+
+// pf_chunk for up to m->pf_wide tokens
+int wide_chunk(qg_model *m, const uint32_t *d_tok, uint32_t ntok, uint32_t s0, bool last)
+{
+    const qg_model_config &c = m->cfg;
+    ihipStream_t *sti = (ihipStream_t *)m->ctx->stream;
+    const uint32_t E = c.embed_dim, H = c.hidden_dim, ldq = m->q_dim + 2 * m->kv_dim;
+    const uint32_t tt = (ntok + qg::kWideTile - 1) / qg::kWideTile;
+    const WideSplit sp = wide_splits(m, tt);
+    const size_t T = (size_t)tt * qg::kWideTile;
+    float *h = m->wd_h[0], *h2 = m->wd_h[1];
+    int rc;
+    // embedding rows into zeroed rows (transformer.rs:74-75, quant.rs:152-174)
+    if ((!whole_rows(m->tok) && qg::launch_fill(h, (size_t)ntok * E, 0.0f, sti)) ||
+        qg::launch_dequantize_rows_dev(m->tok->type, m->tok->d, m->tok->rows, m->tok->cols, d_tok, ntok, h, E, sti))
+        return mfail(m, QG_ERR_HIP, "embedding", hipGetLastError());
+    const size_t kv_layer = (size_t)c.max_seq_len * m->kv_dim;
+    const float scale = 1.0f / sqrtf((float)m->hd);                      // attention.rs:99
+    for (uint32_t l = 0; l < c.n_layers; l++) {
+        // attn_norm of the embeddings, or of h + the previous layer's down
+        if ((rc = wide_planes(m, h, 1, l ? m->wd_fo : nullptr, sp.down, T * E, l ? h2 : nullptr,
+                              m->vec[QG_V_ATTN_NORM][l], E, E, 1, ntok)))
+            return rc;
+        if (l) std::swap(h, h2);
+        const qg::PfMat qkv[3] = {pf_mat(m->w[QG_M_WQ - 2][l], m->wd_qkv),
+                                  pf_mat(m->w[QG_M_WK - 2][l], m->wd_qkv + m->q_dim),
+                                  pf_mat(m->w[QG_M_WV - 2][l], m->wd_qkv + m->q_dim + m->kv_dim)};
+        const bool v_apart = qkv[2].type != qkv[1].type || (qkv[2].g == 1) != (qkv[1].g == 1);
+        const uint32_t s_qk = v_apart ? sp.qk : sp.qkv, s_v = v_apart ? sp.v : sp.qkv;
+        if ((rc = wide_gemm(m, qkv, v_apart ? 2 : 3, E, ntok, ldq, s_qk, T * ldq)) ||
+            (v_apart && (rc = wide_gemm(m, qkv + 2, 1, E, ntok, ldq, s_v, T * ldq))))
+            return rc;
+        float *kc = m->kc + l * kv_layer, *vc = m->vc + l * kv_layer;
+        if (qg::launch_pf_qkv_post(m->wd_qkv, ldq, s_qk, s_v, T * ldq, nullptr, E, c.norm_eps, m->vec[QG_V_BQ][l],
+                                   m->vec[QG_V_BK][l], m->vec[QG_V_BV][l], kc, vc, m->cos_t, m->sin_t, m->q_dim,
+                                   m->kv_dim, m->hd, s0, s0, ntok, sti) ||
+            qg::launch_wide_attention(m->wd_qkv, ldq, kc, vc, m->wd_ao, c.n_heads, m->hd, m->kv_dim, m->n_rep, scale,
+                                      s0, ntok, sti))
+            return mfail(m, QG_ERR_HIP, "prefill attention", hipGetLastError());
+        const qg::PfMat wo = pf_mat(m->w[QG_M_WO - 2][l], m->wd_ao2);
+        if ((rc = wide_planes(m, m->wd_ao, 1, nullptr, 0, 0, nullptr, nullptr, m->q_dim, m->q_dim, 0, ntok)) ||
+            (rc = wide_gemm(m, &wo, 1, m->q_dim, ntok, E, sp.o, T * E)) ||
+            (rc = wide_planes(m, h, 1, m->wd_ao2, sp.o, T * E, h2, m->vec[QG_V_FFN_NORM][l], E, E, 1, ntok)))
+            return rc;
+        std::swap(h, h2);
+        const qg::PfMat gu[2] = {pf_mat(m->w[QG_M_GATE - 2][l], m->wd_g), pf_mat(m->w[QG_M_UP - 2][l], m->wd_g + H)};
+        const qg::PfMat down = pf_mat(m->w[QG_M_DOWN - 2][l], m->wd_fo);
+        if ((rc = wide_gemm(m, gu, 2, E, ntok, 2 * H, sp.gu, T * 2 * H)) ||
+            (rc = wide_planes(m, m->wd_g, sp.gu, m->wd_g + H, sp.gu, T * 2 * H, nullptr, nullptr, H, 2 * (size_t)H, 2,
+                              ntok)) ||
+            (rc = wide_gemm(m, &down, 1, H, ntok, E, sp.down, T * E)))
+            return rc;
+    }
+    return last ? pf_logits(m, h, m->wd_fo, sp.down, T * E, ntok) : QG_OK;
 }
 
 // n tokens at cache slots / positions m->seq ..; leaves the last logits on
@@ -1460,9 +1606,19 @@ int prefill(qg_model *m, const uint32_t *tok, size_t n)
         // the token ids to device once (n <= max_seq_len - seq, checked by the caller)
         QGM_HIP(m, hipMemcpyAsync(m->pf_tok, tok, n * sizeof(uint32_t), hipMemcpyHostToDevice, m->ctx->stream));
         QGM_HIP(m, hipStreamSynchronize(m->ctx->stream));
-        for (size_t i = 0; i < n; i += qg::kPfMaxTokens) {
-            const uint32_t nt = (uint32_t)(n - i < qg::kPfMaxTokens ? n - i : qg::kPfMaxTokens);
-            if ((rc = pf_chunk(m, m->pf_tok + i, nt, (uint32_t)(m->seq + i)))) return rc;
+        // more than one narrow chunk's tokens: wide chunks of equal length (in
+        // whole tiles), where every matrix takes them
+        const bool wide = n > qg::kPfMaxTokens && wide_supported(m);
+        if (wide && (rc = wide_alloc(m))) return rc;
+        size_t len = qg::kPfMaxTokens;
+        if (wide) {
+            const size_t parts = (n + m->pf_wide - 1) / m->pf_wide, per = (n + parts - 1) / parts;
+            len = (per + qg::kWideTile - 1) / qg::kWideTile * qg::kWideTile;
+        }
+        for (size_t i = 0; i < n; i += len) {
+            const uint32_t nt = (uint32_t)std::min(n - i, len);
+            const bool last = i + nt == n;
+            if ((rc = (wide ? wide_chunk : pf_chunk)(m, m->pf_tok + i, nt, (uint32_t)(m->seq + i), last))) return rc;
         }
         m->seq += n;
         return QG_OK;

@@ -1217,7 +1217,7 @@ __global__ void __launch_bounds__(256) pf_qkv_post_k(float *__restrict__ qkv, ui
     const uint32_t pos = pos0 + t, slot = slot0 + t;
     float *q = qkv + (size_t)t * ldq, *k = q + q_dim, *v = k + kv_dim;
     // the GEMM took the norm's numerator: its 1 / rms here, before the biases
-    const float r = pf_inv_rms(ss, ss_ng, t, ss_n, eps);
+    const float r = ss ? pf_inv_rms(ss, ss_ng, t, ss_n, eps) : 1.0f;
     if (i0 < q_dim) {
         const uint32_t j = (i0 % hd) / 2;
         const float c = cos_t[(size_t)pos * half + j], s = sin_t[(size_t)pos * half + j];
@@ -1526,9 +1526,8 @@ int launch_pf_qkv_post(float *qkv, uint32_t ldq, uint32_t ns, uint32_t ns_v, siz
                        uint32_t ntok, ihipStream_t *stream)
 {
     if (ntok == 0) return 0;
-    if (ns < 1 || ns > qgp::kPfMaxSlices || ns_v < 1 || ns_v > qgp::kPfMaxSlices || ntok > kPfMaxTokens ||
-        hd % 2 != 0 || !ss || ss_n == 0 ||
-        ss_n > 0xFFFFFFFFull)
+    if (ns < 1 || ns > qgp::kPfMaxSlices || ns_v < 1 || ns_v > qgp::kPfMaxSlices || ntok > kWideMax ||
+        hd % 2 != 0 || (ss && ss_n == 0) || ss_n > 0xFFFFFFFFull)
         return -1;
     const uint32_t pairs = (q_dim > kv_dim ? q_dim : kv_dim) / 2;
     hipLaunchKernelGGL(qgp::pf_qkv_post_k, dim3((pairs + 255) / 256, ntok), dim3(256), 0, (hipStream_t)stream, qkv,

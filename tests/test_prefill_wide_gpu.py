@@ -1,0 +1,40 @@
+"""GPU parity of the wide batched prefill (prompts of more than 64 tokens,
+rust-inference_amd/csrc/qg_prefill_wide.hip) against the oracle's
+token-by-token forward pass, where its tiles end: prompts around 64 and 128
+tokens, matrices of fewer rows than a tile and of rows that no tile divides,
+rows that start in the middle of a block (cols % 256 == 128), every head size,
+a prompt that takes two wide chunks, and one that continues a cache.  The
+greedy steps after the prompt read every cached position.  Tolerance: DEEP_TOL
+(1e-4 normwise, the bound of the decode and prefill tests)."""
+from __future__ import annotations
+
+import pytest
+
+from test_decode_gpu import DEEP_TOL, SMALL
+from test_prefill_gpu import prefill_and_compare
+
+pytestmark = pytest.mark.gpu
+
+HALF = dict(SMALL, embed_dim=384, n_heads=6, n_kv_heads=2, hidden_dim=640)       # rows of 1.5 and 2.5 blocks
+HD128 = dict(SMALL, embed_dim=512, n_heads=4, n_kv_heads=1, hidden_dim=768)
+HD256 = dict(SMALL, embed_dim=1024, n_heads=4, n_kv_heads=2, hidden_dim=1280)
+
+
+@pytest.mark.parametrize("mix", ["q4_k_m", "q5_k", "q8_0", "q5_k_m"])
+@pytest.mark.parametrize("n", [65, 128, 129])
+def test_tiles(rinf, synth, oracle, ctx, mix, n):
+    e0, errs, _ = prefill_and_compare(rinf, synth, oracle, ctx, SMALL, mix, n, n, 4, 192)
+    assert e0 <= DEEP_TOL and max(errs) <= DEEP_TOL, (e0, errs)
+
+
+@pytest.mark.parametrize("cfg,mix,n", [(HALF, "q4_k_m", 130), (HALF, "q5_k_m", 193), (HALF, "q8_0", 70),
+                                       (HD128, "q4_k_m", 300), (HD256, "q5_k_m", 97), (HD256, "q8_0", 257)])
+def test_shapes(rinf, synth, oracle, ctx, cfg, mix, n):
+    e0, errs, _ = prefill_and_compare(rinf, synth, oracle, ctx, cfg, mix, n, n, 4, 320)
+    assert e0 <= DEEP_TOL and max(errs) <= DEEP_TOL, (e0, errs)
+
+
+def test_two_chunks_and_continued(rinf, synth, oracle, ctx):
+    e0, errs, _ = prefill_and_compare(rinf, synth, oracle, ctx, SMALL, "q4_k_m", 7, 1100, 3, 1200)
+    e1, errs1, _ = prefill_and_compare(rinf, synth, oracle, ctx, SMALL, "q5_k_m", 8, 300, 3, 400, split=81)
+    assert max([e0, e1] + errs + errs1) <= DEEP_TOL, (e0, errs, e1, errs1)
