@@ -198,9 +198,9 @@ int qg_gpu_set_freshness(qg_ctx *ctx, int mode);
  *     within 1e-4 normwise of the reference, but an element far below its
  *     segment's maximum keeps fewer bits (10^4 below: about 8), which shows
  *     where the maxima meet zero weights;
- *   QG_PRECISION_F32: every product rounded to f32 and summed in f32, one
- *     wave per row (the reference's per-product arithmetic, in another
- *     order), at several times the fixed-point kernels' time.
+ *   QG_PRECISION_F32: every product rounded to f32 and summed in f32 (the
+ *     reference's per-product arithmetic, in another order), at several times
+ *     the fixed-point kernels' time.
  * Any other mode: QG_ERR_INVALID_ARG. */
 enum { QG_PRECISION_FIXED22 = 0, QG_PRECISION_F32 = 1 };
 int qg_set_precision(qg_ctx *ctx, int mode);

@@ -864,19 +864,11 @@ int qg_dequant_dev(qg_ctx *ctx, const qg_mat *mat, float *d_out, void *stream)
     if (n == 0) return QG_OK;
     if (!d_out) return fail(ctx, QG_ERR_INVALID_ARG, "out is NULL");
     QG_HIP(ctx, hipSetDevice(ctx->device));
-    uint8_t *w = nullptr;
-    bool temp = false;
-    if ((rc = qg_mat_gguf(ctx, mat, &w, &temp))) return rc;
-    hipStream_t st = pick(ctx, stream);
-    if (qg::launch_dequant(mat->type, w, n, d_out, (ihipStream_t *)st)) {
-        if (temp) (void)hipFree(w);
+    // either layout directly
+    const uint8_t *w = qg_gemv_bytes(mat);
+    if (!w) return fail(ctx, QG_ERR_INVALID_ARG, "matrix holds no device copy");
+    if (qg::launch_dequant(mat->type, mat->plan, w, n, mat->cols, d_out, (ihipStream_t *)pick(ctx, stream)))
         return fail(ctx, QG_ERR_HIP, "dequant launch", hipGetLastError());
-    }
-    if (temp) {                                          // the rebuilt copy lives until the kernel ends
-        const hipError_t e = hipStreamSynchronize(st);
-        (void)hipFree(w);
-        if (e != hipSuccess) return fail(ctx, QG_ERR_HIP, "dequant", e);
-    }
     return QG_OK;
 }
 

@@ -9,7 +9,7 @@
 //   dequant_k<T>      whole-matrix decode to f32, bit-exact (quant.rs:356-840)
 //   deq_row_k<T>      one row with the reference's straddle placement
 //                     (quant.rs:152-174)
-//   gemv_generic<T>   one wave per row, per-element decode; any shape
+//   gemv_quads<T,...>  four elements per lane at a time; any shape, and the f32 mode
 //   gemv_stream<T,..> the fast path: a persistent workgroup stages x once in
 //                     LDS (as fixed-point planes for quant types); a "team"
 //                     of lanes owns whole row groups, each lane one 64-weight
@@ -157,16 +157,159 @@ template <uint32_t T> __device__ __forceinline__ float elem(const uint8_t *b, ui
     return elem_t<T>(b, i);
 }
 
+// ------------------------------------------------- four elements at a time
+//
+// quad<T, RP>(base, ni, e): elements e .. e + 3 (e % 4 == 0) of the GGUF
+// blocks at base, or (RP) of the repacked row group at base (ni items; see
+// repack_k), each the value elem_t gives, bit for bit.  Four neighbours share
+// a block, a scale and a word of codes, and 64 lanes with consecutive quads
+// read a K-quant block's header as one broadcast.
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ uint32_t ldu32(const uint8_t *p)
+{
+    uint32_t v;
+    __builtin_memcpy(&v, p, 4);
+    return v;
+}
+__device__ __forceinline__ uint32_t ldu16(const uint8_t *p)
+{
+    uint16_t v;
+    __builtin_memcpy(&v, p, 2);
+    return v;
+}
+
+template <uint32_t T, bool RP, class IX>
+__device__ __forceinline__ f4 quad(const uint8_t *base, uint32_t ni, IX e)
+{
+    f4 v;
+    if constexpr (T == T_F32) {
+        return *(const f4u *)(base + 4u * e);
+    } else if constexpr (T == T_F16) {
+        const uint32_t a = ldu32(base + 2u * e), b = ldu32(base + 2u * e + 4u);
+        return f4{h2f_exact(a), h2f_exact(a >> 16), h2f_exact(b), h2f_exact(b >> 16)};
+    } else if constexpr (T == T_Q8_0) {
+        const IX blk = e >> 5;
+        const uint32_t i = (uint32_t)e & 31u;
+        uint32_t q;
+        float d;
+        if constexpr (RP) {
+            const uint32_t it = blk >> 1, k = 32u * (blk & 1u) + i;
+            q = ldu32(base + ((k >> 4) * ni + it) * 16u + (k & 15u));
+            d = h2f_exact(ldu16(base + 64u * ni + 2u * blk));
+        } else {
+            const uint8_t *b = base + blk * 34u;
+            q = ldu32(b + 2u + i);
+            d = h2f_exact(ldu16(b));
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = d * (float)(int8_t)(q >> (8 * j));
+    } else if constexpr (T == T_Q4_0) {
+        const uint8_t *b = base + (e >> 5) * 18u;
+        const uint32_t q = ldu16(b + 2u + (((uint32_t)e & 31u) >> 1));      // interleaved nibbles
+        const float d = h2f_exact(ldu16(b));
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = d * (float)((int)((q >> (4 * j)) & 15u) - 8);
+    } else if constexpr (T == T_Q5_0) {
+        const uint8_t *b = base + (e >> 5) * 22u;
+        const uint32_t i = (uint32_t)e & 31u, h = ldu32(b + 2u) >> i;
+        const uint32_t q = ldu32(b + 6u + (i & 15u)) >> (i >= 16u ? 4u : 0u);
+        const float d = h2f_exact(ldu16(b));
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = d * (float)((int)(((q >> (8 * j)) & 15u) | (((h >> j) & 1u) << 4)) - 16);
+    } else if constexpr (T == T_Q4_K || T == T_Q5_K) {
+        const IX blk = e >> 8;
+        const uint32_t j = ((uint32_t)e >> 5) & 7u, l = (uint32_t)e & 31u;
+        const uint8_t *hb = RP ? base + 16u * blk : base + blk * block_bytes(T);
+        uint32_t q;
+        if constexpr (RP && T == T_Q4_K) {
+            const uint32_t it = (uint32_t)e >> 7;
+            q = ldu32(base + 8u * ni + (((j & 2u) + (l >> 4)) * ni + it) * 16u + (l & 15u)) >> (4u * (j & 1u));
+        } else if constexpr (T == T_Q4_K) {
+            q = ldu32(hb + 16u + (j >> 1) * 32u + l) >> (4u * (j & 1u));
+        } else if constexpr (RP) {
+            const uint32_t it = (uint32_t)e >> 6;
+            const uint8_t *c = base + 4u * ni;
+            q = ldu32(c + ((l >> 4) * ni + it) * 16u + (l & 15u)) >> (4u * (j & 1u));
+            const uint32_t w = ldu32(c + 32u * ni + 8u * it + 4u * (l >> 4)) >> (2u * ((l & 15u) >> 2) + (j & 1u));
+            q = (q & 0x0F0F0F0Fu) | ((w & 0x01010101u) << 4);
+        } else {
+            q = ldu32(hb + 48u + (j >> 1) * 32u + l) >> (4u * (j & 1u));
+            q = (q & 0x0F0F0F0Fu) | (((ldu32(hb + 16u + l) >> j) & 0x01010101u) << 4);
+        }
+        if constexpr (T == T_Q4_K) q &= 0x0F0F0F0Fu;
+        const uint4 h = *(const uint4 *)hb;                     // 16-byte aligned: blocks of 144 / 176, heads of 16
+        uint32_t sc, m;
+        k4sm(j, h.y, h.z, h.w, sc, m);
+        const float d1 = h2f_exact(h.x) * (float)sc, m1 = h2f_exact(h.x >> 16) * (float)m;
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = d1 * ub(q, i) - m1;
+    } else {
+        static_assert(T == T_Q6_K, "type");
+        const IX blk = e >> 8;
+        const uint32_t i = (uint32_t)e & 255u, n = i >> 7, k = (i & 127u) >> 5, l = i & 31u;
+        uint32_t ql, qh;
+        float sc, d;
+        if constexpr (RP) {
+            const uint32_t it = 4u * blk + 2u * n + (l >> 4);
+            ql = ldu32(base + ((k & 1u) * ni + it) * 16u + (l & 15u));
+            qh = ldu32(base + (2u * ni + it) * 16u + (l & 15u));
+            sc = (float)(int8_t)base[48u * ni + 4u * it + k];
+            d = h2f_exact(ldu16(base + 52u * ni + 2u * blk));
+        } else {
+            const uint8_t *b = base + blk * 210u;
+            ql = ldu32(b + 64u * n + 32u * (k & 1u) + l);
+            qh = ldu32(b + 128u + 32u * n + l);
+            sc = (float)(int8_t)b[192u + 8u * n + (l >> 4) + 2u * k];
+            d = h2f_exact(ldu16(b + 208u));
+        }
+        const uint32_t q = ((ql >> (4u * (k >> 1))) & 0x0F0F0F0Fu) | (((qh >> (2u * k)) & 0x03030303u) << 4);
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = d * sc * (float)((int)((q >> (8 * j)) & 0xFFu) - 32);
+    }
+    return v;
+}
+
 // ------------------------------------------------------------- dequant
 
-template <uint32_t T>
-__global__ void __launch_bounds__(256) dequant_k(const uint8_t *__restrict__ w, uint64_t n,
-                                                 float *__restrict__ out)
+// ge elements per row group (RP: repacked groups gb bytes apart, ni items;
+// otherwise the whole matrix is one group), n in all; a wave takes 1024
+// consecutive elements of a group, lane l quads l, l + 64, ...  Bound by the f32
+// stores (non-temporal: nothing reads them here): Q4_K 14336 x 4096, 235 MB of
+// them, 38 us, 6.2 TB/s of stores and 7.1 of both (a fill of the same kind
+// reaches 6.9); it was 114 us one element per lane, after rebuilding the GGUF
+// layout in a temporary (64 us).
+template <uint32_t T, bool RP>
+__global__ void __launch_bounds__(256) dequant_k(const uint8_t *__restrict__ w, uint64_t n, uint64_t ge, uint64_t gb,
+                                                 uint32_t ni, uint32_t upg, uint64_t units, float *__restrict__ out)
 {
-    constexpr uint32_t BS = block_elems(T), BB = block_bytes(T);
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t f = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; f < n; f += stride)
-        out[f] = elem<T>(w + (f / BS) * BB, (uint32_t)(f % BS));
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint64_t u = (uint64_t)blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); u < units;
+         u += (uint64_t)gridDim.x * 4u) {
+        const uint32_t grp = RP ? (uint32_t)u / upg : 0u;
+        const uint64_t e0 = (RP ? (uint64_t)((uint32_t)u - grp * upg) : u) * 1024u + 4u * lane;
+        const uint8_t *base = w + grp * gb;
+        const uint64_t f0 = grp * ge;
+        f4 v[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
+            const uint64_t e = e0 + 256u * i;
+            if (e < ge && f0 + e < n) v[i] = RP ? quad<T, RP>(base, ni, (uint32_t)e) : quad<T, RP>(base, ni, e);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
+            const uint64_t e = e0 + 256u * i, f = f0 + e;
+            if (e >= ge || f >= n) continue;
+            if (f + 4u <= n && e + 4u <= ge) {
+                __builtin_nontemporal_store(v[i], (f4u *)(out + f));
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; j++)
+                    if (f + j < n && e + j < ge) out[f + j] = v[i][j];
+            }
+        }
+    }
 }
 
 // quant.rs:152-174: writes only the positions the reference writes.  The
@@ -267,23 +410,99 @@ __device__ __forceinline__ float wave_sum(float v)
     return v;
 }
 
-template <uint32_t T>
-__global__ void __launch_bounds__(256) gemv_generic(const uint8_t *__restrict__ w,
-                                                    const float *__restrict__ x,
-                                                    float *__restrict__ y, uint32_t rows,
-                                                    uint32_t cols)
+// y[r] = sum_c w(r, c) x[c] in f32, from quads: every layout, any cols and any
+// alignment of x.  A row's elements start anywhere in its flat range, so
+// lanes take the aligned quads that cover it and drop what lies outside (by
+// selection: neighbours and padding may hold anything).  FUSE: fused
+// multiply-adds (the general mat-vec); otherwise every product is rounded to
+// f32 before it is added, the reference's arithmetic (quant.rs:195-204).
+//
+// TPR threads per row group of R rows: a wave per row, or (long aligned rows)
+// four waves that share x between four rows.  Bound by the decode's VALU work
+// (K-quants: ~13 instructions per element, the header unpacked per quad).
+// Against one element per lane at a time: F16 3001 x 2050 12.2 -> 4.4 us, Q4_K
+// 4096 x 14336 in the f32 mode 147 -> 34 us.
+struct QuadArgs {
+    const uint8_t *w;
+    const float *x;
+    float *y;
+    uint32_t rows, cols, g, ni;
+    uint64_t gb;
+};
+
+template <uint32_t T, bool RP, bool FUSE, uint32_t TPR, uint32_t R, bool AL>
+__global__ void __launch_bounds__(256) gemv_quads(QuadArgs a)
 {
-    constexpr uint64_t BS = block_elems(T), BB = block_bytes(T);
-    const uint32_t row = blockIdx.x * 4u + threadIdx.x / 64u, lane = threadIdx.x & 63u;
-    if (row >= rows) return;                                    // wave-uniform
-    const uint64_t f0 = (uint64_t)row * cols;
-    float acc = 0.0f;
-    for (uint32_t c = lane; c < cols; c += 64u) {
-        const uint64_t f = f0 + c;
-        acc = __builtin_fmaf(elem<T>(w + (f / BS) * BB, (uint32_t)(f % BS)), x[c], acc);
+    using IX = std::conditional_t<RP, uint32_t, uint64_t>;
+    constexpr uint32_t GPB = 256u / TPR;                         // row groups of R rows per workgroup
+    __shared__ float red[4][R];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x % TPR;
+    const uint32_t r0 = (blockIdx.x * GPB + (TPR == 64u ? wave : 0u)) * R;
+    if (TPR == 64u && r0 >= a.rows) return;                      // wave-uniform
+    const uint8_t *base[R];
+    IX f0[R];
+    float acc[R];
+#pragma unroll
+    for (uint32_t i = 0; i < R; i++) {
+        const uint32_t r = min(r0 + i, a.rows - 1u);
+        base[i] = RP ? a.w + (uint64_t)(r / a.g) * a.gb : a.w;
+        f0[i] = RP ? (IX)(r % a.g) * a.cols : (IX)r * a.cols;
+        acc[i] = 0.f;
     }
-    acc = wave_sum(acc);
-    if (lane == 0) y[row] = acc;
+    auto add = [](float s, float p, float q) { return FUSE ? __builtin_fmaf(p, q, s) : s + p * q; };
+    if constexpr (AL) {                                          // cols % 4 == 0: rows start on quads
+#pragma unroll 4
+        for (uint32_t c = 4u * tid; c < a.cols; c += 4u * TPR) {
+            const f4 x = *(const f4u *)(a.x + c);
+#pragma unroll
+            for (uint32_t i = 0; i < R; i++) {
+                const f4 v = quad<T, RP>(base[i], a.ni, f0[i] + c);
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i] = add(acc[i], v[j], x[j]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (uint32_t i = 0; i < R; i++) {
+            const uint32_t h = (uint32_t)f0[i] & 3u;             // elements of the first quad before the row
+            // the whole quads inside the row, then (lanes 0 and 1) its first
+            // and last quad where they are not
+            const uint32_t q0 = h ? 1u : 0u, q1 = (h + a.cols) / 4u;
+            const float *xr = a.x - h;
+            const IX fa = f0[i] - h;
+#pragma unroll 4
+            for (uint32_t q = q0 + tid; q < q1; q += TPR) {
+                const f4 x = *(const f4u *)(xr + 4u * q);
+                const f4 v = quad<T, RP>(base[i], a.ni, fa + 4u * q);
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i] = add(acc[i], v[j], x[j]);
+            }
+            const uint32_t q = tid == 0u ? 0u : q1;
+            if ((tid == 0u && h) || (tid == 1u && 4u * q1 < h + a.cols && (q1 > 0u || !h))) {
+                const f4 v = quad<T, RP>(base[i], a.ni, fa + 4u * q);
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; j++) {
+                    const uint32_t c = 4u * q + j - h;           // wraps below the row
+                    if (c < a.cols) acc[i] = add(acc[i], v[j], a.x[c]);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < R; i++) acc[i] = wave_sum(acc[i]);
+    if constexpr (TPR == 64u) {
+        if ((threadIdx.x & 63u) == 0u)
+#pragma unroll
+            for (uint32_t i = 0; i < R; i++)
+                if (r0 + i < a.rows) a.y[r0 + i] = acc[i];
+    } else {
+        if ((threadIdx.x & 63u) == 0u)
+#pragma unroll
+            for (uint32_t i = 0; i < R; i++) red[wave][i] = acc[i];
+        __syncthreads();
+        if (threadIdx.x < R && r0 + threadIdx.x < a.rows)
+            a.y[r0 + threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+    }
 }
 
 // ------------------------------------------------- repacked-layout view
@@ -1120,19 +1339,6 @@ __device__ float row_dot_f32(const StreamArgs &a, uint32_t row)
         }
     }
     return wave_sum(acc);
-}
-
-// Plain mat-vec for contexts in QG_PRECISION_F32 (qg_set_precision): one
-// wave per row, row_dot_f32 -- each product w * x rounded to f32 and summed
-// in f32, the reference's arithmetic per product (quant.rs:195-204) in a
-// lane-parallel order -- from the repacked layout (RP) or the GGUF one.
-template <uint32_t T, bool RP>
-__global__ void __launch_bounds__(256) gemv_f32(StreamArgs a)
-{
-    const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (row >= a.rows) return;                                   // wave-uniform
-    const float v = row_dot_f32<T, RP>(a, row);
-    if ((threadIdx.x & 63u) == 0u) a.y[row] = v;
 }
 
 // Per-wave flags "this wave converted a diverting segment" (set before a
@@ -2855,19 +3061,19 @@ int launch_gemv_norm_pair(uint32_t t1, const Plan &p1, const uint8_t *w1, size_t
                                                                                                              : -2;
 }
 
-template <uint32_t T>
-static int launch_generic_t(const uint8_t *w, size_t rows, size_t cols, const float *x, float *y,
-                            hipStream_t st)
+// Long aligned rows share x between four rows of a workgroup where that
+// leaves four waves per SIMD (a row of 4 KB of x is one pass of its 256
+// threads); otherwise a wave per row.
+template <uint32_t T, bool RP, bool FUSE>
+static int launch_quads_t(const QuadArgs &a, hipStream_t st)
 {
-    dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-    hipLaunchKernelGGL((gemv_generic<T>), grid, block, 0, st, w, x, y, (uint32_t)rows,
-                       (uint32_t)cols);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
-template <uint32_t T, bool RP> static int launch_f32_t(const StreamArgs &a, hipStream_t st)
-{
-    hipLaunchKernelGGL((gemv_f32<T, RP>), dim3((a.rows + 3u) / 4u), dim3(256), 0, st, a);
+    const bool al = a.cols % 4u == 0;
+    if (al && a.cols >= 4096u && a.rows >= 4096u)
+        hipLaunchKernelGGL((gemv_quads<T, RP, FUSE, 256, 4, true>), dim3((a.rows + 3u) / 4u), dim3(256), 0, st, a);
+    else if (al)
+        hipLaunchKernelGGL((gemv_quads<T, RP, FUSE, 64, 1, true>), dim3((a.rows + 3u) / 4u), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((gemv_quads<T, RP, FUSE, 64, 1, false>), dim3((a.rows + 3u) / 4u), dim3(256), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -2877,25 +3083,25 @@ int launch_gemv_f32(uint32_t type, const Plan &p, const uint8_t *w, size_t nbyte
     hipStream_t st = (hipStream_t)stream;
     if (rows == 0) return 0;
     if (rows > 0xFFFFFFFFull || cols > 0xFFFFFFFFull || nbytes > 0xFFFFFFFFull) return -1;
-    const StreamArgs a = stream_args(p, w, nbytes, rows, cols, x, y);
+    const QuadArgs a{w, x, y, (uint32_t)rows, (uint32_t)cols, p.rp ? p.g : 1u, p.ni, p.group_bytes};
     if (p.rp) {
         switch (type) {
-        case T_Q8_0: return launch_f32_t<T_Q8_0, true>(a, st);
-        case T_Q4_K: return launch_f32_t<T_Q4_K, true>(a, st);
-        case T_Q5_K: return launch_f32_t<T_Q5_K, true>(a, st);
-        case T_Q6_K: return launch_f32_t<T_Q6_K, true>(a, st);
+        case T_Q8_0: return launch_quads_t<T_Q8_0, true, false>(a, st);
+        case T_Q4_K: return launch_quads_t<T_Q4_K, true, false>(a, st);
+        case T_Q5_K: return launch_quads_t<T_Q5_K, true, false>(a, st);
+        case T_Q6_K: return launch_quads_t<T_Q6_K, true, false>(a, st);
         default: return -1;
         }
     }
     switch (type) {
-    case T_F32: return launch_f32_t<T_F32, false>(a, st);
-    case T_F16: return launch_f32_t<T_F16, false>(a, st);
-    case T_Q4_0: return launch_f32_t<T_Q4_0, false>(a, st);
-    case T_Q5_0: return launch_f32_t<T_Q5_0, false>(a, st);
-    case T_Q8_0: return launch_f32_t<T_Q8_0, false>(a, st);
-    case T_Q4_K: return launch_f32_t<T_Q4_K, false>(a, st);
-    case T_Q5_K: return launch_f32_t<T_Q5_K, false>(a, st);
-    case T_Q6_K: return launch_f32_t<T_Q6_K, false>(a, st);
+    case T_F32: return launch_quads_t<T_F32, false, false>(a, st);
+    case T_F16: return launch_quads_t<T_F16, false, false>(a, st);
+    case T_Q4_0: return launch_quads_t<T_Q4_0, false, false>(a, st);
+    case T_Q5_0: return launch_quads_t<T_Q5_0, false, false>(a, st);
+    case T_Q8_0: return launch_quads_t<T_Q8_0, false, false>(a, st);
+    case T_Q4_K: return launch_quads_t<T_Q4_K, false, false>(a, st);
+    case T_Q5_K: return launch_quads_t<T_Q5_K, false, false>(a, st);
+    case T_Q6_K: return launch_quads_t<T_Q6_K, false, false>(a, st);
     default: return -1;
     }
 }
@@ -2906,15 +3112,16 @@ int launch_gemv_generic(uint32_t type, const uint8_t *w, size_t rows, size_t col
     hipStream_t st = (hipStream_t)stream;
     if (rows == 0) return 0;
     if (rows > 0xFFFFFFFFull || cols > 0xFFFFFFFFull) return -1;
+    const QuadArgs a{w, x, y, (uint32_t)rows, (uint32_t)cols, 1u, 0u, 0u};
     switch (type) {
-    case T_F32: return launch_generic_t<T_F32>(w, rows, cols, x, y, st);
-    case T_F16: return launch_generic_t<T_F16>(w, rows, cols, x, y, st);
-    case T_Q4_0: return launch_generic_t<T_Q4_0>(w, rows, cols, x, y, st);
-    case T_Q5_0: return launch_generic_t<T_Q5_0>(w, rows, cols, x, y, st);
-    case T_Q8_0: return launch_generic_t<T_Q8_0>(w, rows, cols, x, y, st);
-    case T_Q4_K: return launch_generic_t<T_Q4_K>(w, rows, cols, x, y, st);
-    case T_Q5_K: return launch_generic_t<T_Q5_K>(w, rows, cols, x, y, st);
-    case T_Q6_K: return launch_generic_t<T_Q6_K>(w, rows, cols, x, y, st);
+    case T_F32: return launch_quads_t<T_F32, false, true>(a, st);
+    case T_F16: return launch_quads_t<T_F16, false, true>(a, st);
+    case T_Q4_0: return launch_quads_t<T_Q4_0, false, true>(a, st);
+    case T_Q5_0: return launch_quads_t<T_Q5_0, false, true>(a, st);
+    case T_Q8_0: return launch_quads_t<T_Q8_0, false, true>(a, st);
+    case T_Q4_K: return launch_quads_t<T_Q4_K, false, true>(a, st);
+    case T_Q5_K: return launch_quads_t<T_Q5_K, false, true>(a, st);
+    case T_Q6_K: return launch_quads_t<T_Q6_K, false, true>(a, st);
     default: return -1;
     }
 }
@@ -2925,26 +3132,42 @@ static unsigned grid_for(uint64_t n)
     return (unsigned)(g < 1 ? 1 : g > 65536 ? 65536 : g);
 }
 
-template <uint32_t T>
-static int launch_dequant_t(const uint8_t *w, size_t n, float *out, hipStream_t st)
+template <uint32_t T, bool RP>
+static int launch_dequant_t(const Plan &p, const uint8_t *w, size_t n, size_t cols, float *out, hipStream_t st)
 {
-    hipLaunchKernelGGL((dequant_k<T>), dim3(grid_for(n)), dim3(256), 0, st, w, (uint64_t)n, out);
+    const uint64_t ge = RP ? (uint64_t)p.g * cols : (uint64_t)n;
+    const uint32_t upg = RP ? (uint32_t)((ge + 1023u) / 1024u) : 0u;
+    const uint64_t units = RP ? (uint64_t)p.n_groups * upg : (ge + 1023u) / 1024u;
+    if (units > 0xFFFFFFFFull) return -1;                        // more than 2^42 elements
+    const uint64_t wgs = (units + 3u) / 4u;
+    hipLaunchKernelGGL((dequant_k<T, RP>), dim3((unsigned)(wgs < 65536u ? wgs : 65536u)), dim3(256), 0, st, w,
+                       (uint64_t)n, ge, RP ? p.group_bytes : 0u, RP ? p.ni : 0u, upg, units, out);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_dequant(uint32_t type, const uint8_t *w, size_t n, float *out, ihipStream_t *stream)
+int launch_dequant(uint32_t type, const Plan &p, const uint8_t *w, size_t n, size_t cols, float *out,
+                   ihipStream_t *stream)
 {
     hipStream_t st = (hipStream_t)stream;
     if (n == 0) return 0;
+    if (p.rp) {
+        switch (type) {
+        case T_Q8_0: return launch_dequant_t<T_Q8_0, true>(p, w, n, cols, out, st);
+        case T_Q4_K: return launch_dequant_t<T_Q4_K, true>(p, w, n, cols, out, st);
+        case T_Q5_K: return launch_dequant_t<T_Q5_K, true>(p, w, n, cols, out, st);
+        case T_Q6_K: return launch_dequant_t<T_Q6_K, true>(p, w, n, cols, out, st);
+        default: return -1;
+        }
+    }
     switch (type) {
-    case T_F32: return launch_dequant_t<T_F32>(w, n, out, st);
-    case T_F16: return launch_dequant_t<T_F16>(w, n, out, st);
-    case T_Q4_0: return launch_dequant_t<T_Q4_0>(w, n, out, st);
-    case T_Q5_0: return launch_dequant_t<T_Q5_0>(w, n, out, st);
-    case T_Q8_0: return launch_dequant_t<T_Q8_0>(w, n, out, st);
-    case T_Q4_K: return launch_dequant_t<T_Q4_K>(w, n, out, st);
-    case T_Q5_K: return launch_dequant_t<T_Q5_K>(w, n, out, st);
-    case T_Q6_K: return launch_dequant_t<T_Q6_K>(w, n, out, st);
+    case T_F32: return launch_dequant_t<T_F32, false>(p, w, n, cols, out, st);
+    case T_F16: return launch_dequant_t<T_F16, false>(p, w, n, cols, out, st);
+    case T_Q4_0: return launch_dequant_t<T_Q4_0, false>(p, w, n, cols, out, st);
+    case T_Q5_0: return launch_dequant_t<T_Q5_0, false>(p, w, n, cols, out, st);
+    case T_Q8_0: return launch_dequant_t<T_Q8_0, false>(p, w, n, cols, out, st);
+    case T_Q4_K: return launch_dequant_t<T_Q4_K, false>(p, w, n, cols, out, st);
+    case T_Q5_K: return launch_dequant_t<T_Q5_K, false>(p, w, n, cols, out, st);
+    case T_Q6_K: return launch_dequant_t<T_Q6_K, false>(p, w, n, cols, out, st);
     default: return -1;
     }
 }
