@@ -46,13 +46,14 @@ constexpr uint32_t kRecentMax = 64;       // model.rs:370-374 passes the last 64
 constexpr uint32_t kSampleWG = 256;       // partial-argmax workgroups
 constexpr uint32_t kMaxGroup = 8;         // query heads per attention workgroup
 constexpr uint32_t kMaxSplit = 64;        // position ranges per head
-constexpr uint32_t kMinLen = 8;           // positions per range (the last may hold fewer)
+constexpr uint32_t kRangeTile = 64;       // positions a workgroup takes at a time (16 per wave)
 
-// Positions per range for seq cached positions; ranges = ceil(seq / len).
+// Positions per range for seq cached positions (whole tiles; the last range
+// may hold fewer); ranges = ceil(seq / len) <= nsplit.
 __host__ __device__ __forceinline__ uint32_t range_len(uint32_t seq, uint32_t nsplit)
 {
-    const uint32_t l = (seq + nsplit - 1) / nsplit;
-    return l > kMinLen ? l : kMinLen;
+    const uint32_t t = (seq + kRangeTile - 1) / kRangeTile;
+    return (t + nsplit - 1) / nsplit * kRangeTile;
 }
 
 // Per-token state read by the kernels: the token fed to the next forward
@@ -182,167 +183,192 @@ __device__ __forceinline__ float rope1(float self, float other, uint32_t d, floa
     return p0 + ((d & 1u) ? p1 : -p1);
 }
 
-// Attention of the token at st->pos over positions [j0, j1) of the
-// seq = slot + 1 cached ones, for the `grp` query heads h0 .. h0 + grp - 1
-// that share one kv head (head_dim = 64 * E), with the projections'
-// post-processing folded in: q, k, v biases (attention.rs:66-76), RoPE of q
-// and k (attention.rs:78-87) and the cache append at `slot`
-// (attention.rs:89-90, kv_cache.rs:52-73).  The range that holds `slot` uses
-// this token's k and v from registers, and its first head group of each kv
-// head stores them to the cache, so no other workgroup reads the slot being
-// written.
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// Maximum / sum over the 16 lanes of a row, to all of them.
+__device__ __forceinline__ float row_max(float v)
+{
+    v = fmaxf(v, dppf<0xB1>(v, v));
+    v = fmaxf(v, dppf<0x4E>(v, v));
+    v = fmaxf(v, dppf<0x141>(v, v));
+    return fmaxf(v, dppf<0x140>(v, v));
+}
+__device__ __forceinline__ float row_sum(float v)
+{
+    v += dppf<0xB1>(v, 0.f);
+    v += dppf<0x4E>(v, 0.f);
+    v += dppf<0x141>(v, 0.f);
+    return v + dppf<0x140>(v, 0.f);
+}
+
+// Elements d .. d + 3 (d % 4 == 0) of a head after RoPE: the pairs (0, 1) and
+// (2, 3) turned by the position's c, s (rows of the tables, at d / 2).  The
+// same expressions as rope1.
+__device__ __forceinline__ v4f rope4(v4f x, float2 c, float2 s)
+{
+    const float a0 = x[0] * c.x, b0 = x[1] * s.x, a1 = x[1] * c.x, b1 = x[0] * s.x;
+    const float a2 = x[2] * c.y, b2 = x[3] * s.y, a3 = x[3] * c.y, b3 = x[2] * s.y;
+    return v4f{a0 - b0, a1 + b1, a2 - b2, a3 + b3};
+}
+
+// Attention of the token at st->pos over one range of the seq = slot + 1
+// cached positions, for the `grp` (at most 8) query heads h0 .. that share one
+// kv head (head_dim = 64 * E), with the projections' post-processing folded
+// in: q, k, v biases (attention.rs:66-76), RoPE of q and k (attention.rs:78-87)
+// and the cache append at `slot` (attention.rs:89-90, kv_cache.rs:52-73).  The
+// range that holds `slot` uses this token's k and v from registers, and its
+// first head group of each kv head stores them to the cache, so no other
+// workgroup reads the slot being written.
 //
-// (Merging the ranges in the last workgroup to finish, behind a device-scope
-// counter, measured slower than the separate merge kernel: the fences that
-// make the partial sums visible across the XCDs' L2 caches cost more than the
-// launch.)
+// Workgroup (head group, range): four waves, each 16 positions of every tile
+// of 64, on the f32 matrix cores (v_mfma_f32_16x16x4f32: f32 products and
+// sums; 8 of the 16 rows at most are heads, and it is still latency and not the
+// matrix rate that bounds the kernel).  All of a tile's K and V rows are
+// requested before any is used.  S = Q K^T: 4 HD / 16 MFMAs, lane (c, g) holding
+// elements 16 k + 4 g .. + 4 of head c and of position c (an MFMA's four
+// k-steps are the lane's four elements); P = exp(S - m) goes through the wave's
+// LDS rows into the A layout; P V: lane (c, g) holds columns 64 b + 4 c .. + 4
+// of positions 4 g + j, so tile (b, e)'s column c is 64 b + 4 c + e.  The four
+// waves are merged in LDS.  Writes the unnormalised partial output sum_j
+// exp(s_j - m) v_j and (m, l = sum_j exp(s_j - m)) of the range; workgroups
+// whose range starts past seq exit.
 //
-// Workgroup (head group, range): 4 waves, each lane owns dimensions
-// lane + 64 e (every K and V row is one coalesced read shared by the group's
-// heads).  A wave takes positions j0 + wave + 4 p in chunks of kPW, all K and
-// V rows of a chunk loaded before any use, with a running (max, sum, output)
-// per head (the softmax of attention.rs:101-119 over the wave's positions);
-// the four waves are merged in LDS.  Writes the unnormalised partial output
-// sum_j exp(s_j - m) v_j and (m, l = sum_j exp(s_j - m)) of the range;
-// workgroups whose range starts past seq exit.
-// Positions per wave per chunk: the chunk's code is unrolled over heads and
-// positions, and a larger chunk made the kernel slower (straight-line code
-// fetched cold by every workgroup) while short ranges fill only one chunk.
-constexpr uint32_t kPW = 2;
+// Qwen2-7B heads (28 over 4) at 2000-2256 positions: SPLIT_US us a layer where
+// one position and head at a time on the VALU (a 64-lane sum for every score)
+// took 15.6, and the merge COMB_US us (6.7).  (Merging the ranges in the last
+// workgroup to finish, behind a device-scope counter, measured slower than the
+// separate merge kernel: the fences that make the partial sums visible across
+// the XCDs' L2 caches cost more than the launch.)
 template <int E>
 __global__ void __launch_bounds__(256) attn_rope_split_k(AttnArgs a)
 {
-    constexpr uint32_t HD = 64 * E;
+    constexpr uint32_t HD = 64 * E, KS = HD / 16u;
     __shared__ float sacc[4][kMaxGroup][HD];
     __shared__ float sml[4][kMaxGroup][2];
-    // wave index as a uniform value: the position loop's bounds depend on it,
-    // and a per-lane value would turn every branch on them into exec masking
+    __shared__ float sp[4][16][20];
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t c = lane & 15u, g = lane >> 4;
     const uint32_t grp = a.grp, split = blockIdx.x % a.nsplit, h0 = (blockIdx.x / a.nsplit) * grp;
     const uint32_t kvo = (h0 / a.n_rep) * HD;
-    // Every load below is unconditional (clamped indices, selects after the
-    // loads): a load behind a branch waits for everything issued before it.
-    // The projections do not depend on the step record, so they are in flight
-    // while it arrives.
-    float qv[kMaxGroup][E], kn[E], vn[E];
+    // the projections do not depend on the step record: in flight while it arrives
+    const uint32_t qo = (h0 + (c < grp ? c : 0u)) * HD + 4u * g, ko = kvo + 4u * g;
+    v4f qa[KS], kn[KS], vn[E];
 #pragma unroll
-    for (uint32_t r = 0; r < kMaxGroup; r++)
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            const uint32_t i = (h0 + (r < grp ? r : 0u)) * HD + lane + 64 * e;
-            qv[r][e] = a.q[i] + a.bq[i];
-        }
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        kn[e] = a.k[kvo + lane + 64 * e] + a.bk[kvo + lane + 64 * e];
-        vn[e] = a.v[kvo + lane + 64 * e] + a.bv[kvo + lane + 64 * e];
+    for (uint32_t k = 0; k < KS; k++) {
+        qa[k] = *(const v4f *)(a.q + qo + 16u * k) + *(const v4f *)(a.bq + qo + 16u * k);
+        kn[k] = *(const v4f *)(a.k + ko + 16u * k) + *(const v4f *)(a.bk + ko + 16u * k);
     }
+#pragma unroll
+    for (int b = 0; b < E; b++)
+        vn[b] = *(const v4f *)(a.v + kvo + 64u * b + 4u * c) + *(const v4f *)(a.bv + kvo + 64u * b + 4u * c);
     const uint32_t pos = a.st->pos, slot = a.st->slot, seq = slot + 1;
-    const uint32_t len = range_len(seq, a.nsplit);
-    const uint32_t j0 = split * len, j1 = min(seq, j0 + len);
-    // K and V rows of this wave's positions j0 + wave + 4 p, kPW at a time,
-    // clamped into the cache rows that exist (a workgroup past seq loads and
-    // exits); the next chunk is in flight while one is used
-    float kk[kPW][E], vv[kPW][E], nk[kPW][E], nv[kPW][E];
-    auto load = [&](uint32_t b, float (&ko)[kPW][E], float (&vo)[kPW][E]) {
+    const uint32_t len = range_len(seq, a.nsplit), j0 = split * len, j1 = min(seq, j0 + len);
+    if (j0 >= seq) return;
+    // K and V rows of the 16 positions at base, clamped into the rows that exist
+    v4f kk[KS], vv[4][E];
+    auto load = [&](uint32_t base) {
+        const float *kr = a.kc + (size_t)min(base + c, slot) * a.kv_dim + ko;
 #pragma unroll
-        for (uint32_t p = 0; p < kPW; p++) {
-            const uint32_t j = min(b + 4 * p, slot);
-            const float *kr = a.kc + (size_t)j * a.kv_dim + kvo, *vr = a.vc + (size_t)j * a.kv_dim + kvo;
+        for (uint32_t k = 0; k < KS; k++) kk[k] = *(const v4f *)(kr + 16u * k);
 #pragma unroll
-            for (int e = 0; e < E; e++) {
-                ko[p][e] = kr[lane + 64 * e];
-                vo[p][e] = vr[lane + 64 * e];
-            }
+        for (uint32_t j = 0; j < 4; j++) {
+            const float *vr = a.vc + (size_t)min(base + 4u * g + j, slot) * a.kv_dim + kvo + 4u * c;
+#pragma unroll
+            for (int b = 0; b < E; b++) vv[j][b] = *(const v4f *)(vr + 64u * b);
         }
     };
-    uint32_t base = j0 + wave;
-    load(base, kk, vv);
-    // cos / sin of this lane's pairs (the table rows of `pos`)
-    float cv[E], sv[E];
+    uint32_t base = j0 + 16u * wave;
+    load(base);
+    {
+        const float *ct = a.cos_t + (size_t)pos * (HD / 2) + 2u * g, *sn = a.sin_t + (size_t)pos * (HD / 2) + 2u * g;
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-        cv[e] = a.cos_t[(size_t)pos * (HD / 2) + ((lane + 64 * e) >> 1)];
-        sv[e] = a.sin_t[(size_t)pos * (HD / 2) + ((lane + 64 * e) >> 1)];
-    }
-#pragma unroll
-    for (uint32_t r = 0; r < kMaxGroup; r++)
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            const float o = __shfl_xor(qv[r][e], 1, 64);
-            qv[r][e] = r < grp ? rope1(qv[r][e], o, lane + 64 * e, cv[e], sv[e]) : 0.f;
-        }
-#pragma unroll
-    for (int e = 0; e < E; e++) kn[e] = rope1(kn[e], __shfl_xor(kn[e], 1, 64), lane + 64 * e, cv[e], sv[e]);
-    if (j0 >= seq) return;
-    const bool has_new = j1 == seq;
-    if (has_new && h0 % a.n_rep == 0 && wave == 0) {
-        float *kr = a.kc + (size_t)slot * a.kv_dim + kvo, *vr = a.vc + (size_t)slot * a.kv_dim + kvo;
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            kr[lane + 64 * e] = kn[e];
-            vr[lane + 64 * e] = vn[e];
+        for (uint32_t k = 0; k < KS; k++) {
+            const float2 cv = *(const float2 *)(ct + 8u * k), sv = *(const float2 *)(sn + 8u * k);
+            qa[k] = rope4(qa[k], cv, sv);
+            kn[k] = rope4(kn[k], cv, sv);
         }
     }
-    float m[kMaxGroup], l[kMaxGroup], acc[kMaxGroup][E];
+    if (j1 == seq && h0 % a.n_rep == 0 && wave == 0) {
+        float *kr = a.kc + (size_t)slot * a.kv_dim + ko, *vr = a.vc + (size_t)slot * a.kv_dim + kvo + 4u * c;
+        if (c == 0)
 #pragma unroll
-    for (uint32_t r = 0; r < kMaxGroup; r++) {
-        m[r] = -INFINITY;
-        l[r] = 0.f;
+            for (uint32_t k = 0; k < KS; k++) *(v4f *)(kr + 16u * k) = kn[k];
+        if (g == 0)
 #pragma unroll
-        for (int e = 0; e < E; e++) acc[r][e] = 0.f;
+            for (int b = 0; b < E; b++) *(v4f *)(vr + 64u * b) = vn[b];
     }
-    for (; base < j1; base += 4 * kPW) {
-        const uint32_t np = min((j1 - base + 3) / 4, kPW);   // this wave's positions in the chunk
-        if (base + 4 * kPW < j1) load(base + 4 * kPW, nk, nv);
-        // the slot being appended comes from registers (its cache row is written above)
+    // of heads 4 g + i
+    float m[4], l[4];
+    v4f o[E][4];
 #pragma unroll
-        for (uint32_t p = 0; p < kPW; p++)
-            if (base + 4 * p == slot)
+    for (uint32_t i = 0; i < 4; i++) { m[i] = -INFINITY; l[i] = 0.f; }
 #pragma unroll
-                for (int e = 0; e < E; e++) { kk[p][e] = kn[e]; vv[p][e] = vn[e]; }
+    for (int b = 0; b < E; b++)
 #pragma unroll
-        for (uint32_t r = 0; r < kMaxGroup; r++) {
-            if (r >= grp) break;
-            float sc[kPW], cm = -INFINITY;
+        for (int e = 0; e < 4; e++) o[b][e] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (; base < j1; base += kRangeTile) {
+        // the slot being appended comes from registers (and stands in for the
+        // masked positions after it, whose clamped row may hold anything)
+        if (base + 16u > slot) {
 #pragma unroll
-            for (uint32_t p = 0; p < kPW; p++) {
-                if (p >= np) break;
-                float t = 0.f;
+            for (uint32_t k = 0; k < KS; k++)
 #pragma unroll
-                for (int e = 0; e < E; e++) t += qv[r][e] * kk[p][e];
-                sc[p] = wave_sum(t) * a.scale;
-                cm = fmaxf(cm, sc[p]);
+                for (int e = 0; e < 4; e++) kk[k][e] = base + c >= slot ? kn[k][e] : kk[k][e];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+#pragma unroll
+                for (int b = 0; b < E; b++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) vv[j][b][e] = base + 4u * g + j >= slot ? vn[b][e] : vv[j][b][e];
+        }
+        v4f s = v4f{0.f, 0.f, 0.f, 0.f}, s2 = s;
+#pragma unroll
+        for (uint32_t k = 0; k < KS; k += 2) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                s = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[k][e], kk[k][e], s, 0, 0, 0);
+                s2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[k + 1][e], kk[k + 1][e], s2, 0, 0, 0);
             }
-            const float mn = fmaxf(m[r], cm);
-            const float al = m[r] == -INFINITY ? 0.f : expf(m[r] - mn);
-            float ls = 0.f, o[E];
-#pragma unroll
-            for (int e = 0; e < E; e++) o[e] = 0.f;
-#pragma unroll
-            for (uint32_t p = 0; p < kPW; p++) {
-                if (p >= np) break;
-                const float ex = expf(sc[p] - mn);
-                ls += ex;
-#pragma unroll
-                for (int e = 0; e < E; e++) o[e] += ex * vv[p][e];
-            }
-            l[r] = l[r] * al + ls;
-#pragma unroll
-            for (int e = 0; e < E; e++) acc[r][e] = acc[r][e] * al + o[e];
-            m[r] = mn;
         }
+        float al[4];
 #pragma unroll
-        for (uint32_t p = 0; p < kPW; p++)
+        for (uint32_t i = 0; i < 4; i++) {
+            const float sc = base + c < j1 ? (s[i] + s2[i]) * a.scale : -INFINITY;
+            const float mn = fmaxf(m[i], row_max(sc));          // finite: the tile's first position is cached
+            al[i] = m[i] == -INFINITY ? 0.f : expf(m[i] - mn);
+            const float p = expf(sc - mn);
+            m[i] = mn;
+            l[i] = l[i] * al[i] + p;
+            sp[wave][4u * g + i][c] = p;
+        }
+        __builtin_amdgcn_wave_barrier();
+        const v4f pa = *(const v4f *)&sp[wave][c][4u * g];
 #pragma unroll
-            for (int e = 0; e < E; e++) { kk[p][e] = nk[p][e]; vv[p][e] = nv[p][e]; }
+        for (int b = 0; b < E; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[b][e][i] *= al[i];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++)
+#pragma unroll
+            for (int b = 0; b < E; b++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    o[b][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[j], vv[j][b][e], o[b][e], 0, 0, 0);
+        __builtin_amdgcn_wave_barrier();
+        if (base + kRangeTile < j1) load(base + kRangeTile);
     }
 #pragma unroll
-    for (uint32_t r = 0; r < kMaxGroup; r++) {
-        if (r >= grp) break;
+    for (uint32_t i = 0; i < 4; i++) {
+        const uint32_t r = 4u * g + i;
+        const float ls = row_sum(l[i]);
+        if (r < grp) {
 #pragma unroll
-        for (int e = 0; e < E; e++) sacc[wave][r][lane + 64 * e] = acc[r][e];
-        if (lane == 0) { sml[wave][r][0] = m[r]; sml[wave][r][1] = l[r]; }
+            for (int b = 0; b < E; b++)
+                *(v4f *)&sacc[wave][r][64u * b + 4u * c] = v4f{o[b][0][i], o[b][1][i], o[b][2][i], o[b][3][i]};
+            if (c == 0) { sml[wave][r][0] = m[i]; sml[wave][r][1] = ls; }
+        }
     }
     __syncthreads();
     // merge the waves: weights exp(m_w - M) (0 for a wave without positions)
@@ -359,40 +385,54 @@ __global__ void __launch_bounds__(256) attn_rope_split_k(AttnArgs a)
             sum += f * sacc[w][r][d];
             lsum += f * sml[w][r][1];
         }
-        const size_t o = (size_t)(h0 + r) * a.nsplit + split;
-        a.part[o * HD + d] = sum;
+        const size_t po = (size_t)(h0 + r) * a.nsplit + split;
+        a.part[po * HD + d] = sum;
         if (d == 0) {
-            a.ml[2 * o] = mx;
-            a.ml[2 * o + 1] = lsum;
+            a.ml[2 * po] = mx;
+            a.ml[2 * po + 1] = lsum;
         }
     }
 }
 
 // out[h] = sum_s w_s part_s with w_s = exp(m_s - max m) / sum_s exp(m_s - max m) l_s:
-// the softmax-weighted sum of v over all positions.  One workgroup per head;
-// wave 0 derives the weights of the ranges in use.
-__global__ void __launch_bounds__(256) attn_combine_k(const float *__restrict__ part, const float *__restrict__ ml,
-                                                      float *__restrict__ out, const Step *__restrict__ st,
-                                                      uint32_t hd, uint32_t nsplit)
+// the softmax-weighted sum of v over all positions.  One workgroup of 1024
+// threads per head: wave w takes dimensions 64 (w % E) .. of the ranges s = w / E
+// (mod 16 / E), all of them requested at once (clamped to the ranges in use;
+// those need the step record only for their number), and derives the ranges'
+// weights itself, one per lane.
+template <int E>
+__global__ void __launch_bounds__(1024) attn_combine_k(const float *__restrict__ part, const float *__restrict__ ml,
+                                                       float *__restrict__ out, const Step *__restrict__ st,
+                                                       uint32_t nsplit)
 {
-    __shared__ float wt[kMaxSplit];
-    const uint32_t h = blockIdx.x, seq = st->slot + 1;
-    const uint32_t len = range_len(seq, nsplit), nr = (seq + len - 1) / len;
-    const float *m = ml + (size_t)h * nsplit * 2;
-    if (threadIdx.x < 64) {
-        const uint32_t s = threadIdx.x;
-        const float ms = s < nr ? m[2 * s] : -INFINITY, ls = s < nr ? m[2 * s + 1] : 0.f;
-        const float mx = wave_max(ms);
-        const float w = s < nr ? expf(ms - mx) : 0.f;
-        const float l = wave_sum(w * ls);
-        wt[s] = w / l;
+    constexpr uint32_t HD = 64 * E, NW = 16u / E, PER = kMaxSplit / NW;
+    __shared__ float red[NW][HD];
+    const uint32_t h = blockIdx.x, lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t d = 64u * (wave % E) + lane, s0 = wave / E;
+    const float *p = part + (size_t)h * nsplit * HD + d;
+    const float2 v = *(const float2 *)(ml + 2u * ((size_t)h * nsplit + min(lane, nsplit - 1u)));
+    float u[PER];
+#pragma unroll
+    for (uint32_t i = 0; i < PER; i++) u[i] = p[(size_t)min(s0 + i * NW, nsplit - 1u) * HD];
+    const uint32_t seq = st->slot + 1, len = range_len(seq, nsplit), nr = (seq + len - 1) / len;
+    const float ms = lane < nr ? v.x : -INFINITY;
+    const float mx = wave_max(ms);
+    const float w = lane < nr ? expf(ms - mx) : 0.f;
+    const float wt = w / wave_sum(lane < nr ? w * v.y : 0.f);
+    float acc = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < PER; i++) {
+        const uint32_t s = s0 + i * NW;
+        const float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wt), (int)s));
+        acc += s < nr ? f * u[i] : 0.f;
     }
+    red[s0][d] = acc;
     __syncthreads();
-    const float *p = part + (size_t)h * nsplit * hd;
-    for (uint32_t d = threadIdx.x; d < hd; d += blockDim.x) {
-        float acc = 0.f;
-        for (uint32_t s = 0; s < nr; s++) acc += wt[s] * p[(size_t)s * hd + d];
-        out[h * hd + d] = acc;
+    if (threadIdx.x < HD) {
+        float t = 0.f;
+#pragma unroll
+        for (uint32_t i = 0; i < NW; i++) t += red[i][threadIdx.x];
+        out[h * HD + threadIdx.x] = t;
     }
 }
 
@@ -1143,8 +1183,16 @@ int enqueue_forward(qg_model *m)
                     hipLaunchKernelGGL(qgm::attn_rope_split_k<2>, grid, dim3(256), 0, st, aa);
                 else
                     hipLaunchKernelGGL(qgm::attn_rope_split_k<4>, grid, dim3(256), 0, st, aa);
-                hipLaunchKernelGGL(qgm::attn_combine_k, dim3(c.n_heads), dim3(256), 0, st, m->att_part, m->att_ml,
-                                   m->ao, m->d_step, m->hd, m->att_nsplit);
+                const dim3 cg(c.n_heads), cb(1024);
+                if (m->hd == 64)
+                    hipLaunchKernelGGL(qgm::attn_combine_k<1>, cg, cb, 0, st, m->att_part, m->att_ml, m->ao, m->d_step,
+                                       m->att_nsplit);
+                else if (m->hd == 128)
+                    hipLaunchKernelGGL(qgm::attn_combine_k<2>, cg, cb, 0, st, m->att_part, m->att_ml, m->ao, m->d_step,
+                                       m->att_nsplit);
+                else
+                    hipLaunchKernelGGL(qgm::attn_combine_k<4>, cg, cb, 0, st, m->att_part, m->att_ml, m->ao, m->d_step,
+                                       m->att_nsplit);
             }
         } else {
             hipLaunchKernelGGL(qgm::qkv_post_k, dim3((pairs + 255) / 256), dim3(256), 0, st, m->q, m->k, m->v,
@@ -1656,18 +1704,15 @@ int qg_model_create(qg_ctx *ctx, const qg_model_config *cfg, qg_model **out)
     m->kv_dim = n_kv * hd;
     m->n_rep = c.n_heads / n_kv;
     // attention layout: workgroups of grp query heads (a divisor of n_rep, at
-    // most 8) times up to 64 position ranges of at least 8 positions, about
-    // 256 workgroups in all at long sequences; any max_seq_len
+    // most 8) times up to 64 position ranges of whole tiles of 64 positions;
+    // any max_seq_len
     constexpr size_t kLdsMax = 65536;
     if (hd == 64 || hd == 128 || hd == 256) {
         uint32_t grp = 1;
         for (uint32_t d = 1; d <= qgm::kMaxGroup; d++)
             if (m->n_rep % d == 0) grp = d;
-        const uint32_t groups = c.n_heads / grp;
-        uint32_t ns = (256 + groups - 1) / groups;
-        ns = ns < 1 ? 1 : ns > qgm::kMaxSplit ? qgm::kMaxSplit : ns;
         m->att_grp = grp;
-        m->att_nsplit = ns;
+        m->att_nsplit = qgm::kMaxSplit;
     } else {
         m->att_lds = ((size_t)hd + c.max_seq_len) * sizeof(float);
         if (m->att_lds > kLdsMax) {
