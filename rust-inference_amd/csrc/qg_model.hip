@@ -233,9 +233,9 @@ __device__ __forceinline__ v4f rope4(v4f x, float2 c, float2 s)
 // exp(s_j - m) v_j and (m, l = sum_j exp(s_j - m)) of the range; workgroups
 // whose range starts past seq exit.
 //
-// Qwen2-7B heads (28 over 4) at 2000-2256 positions: SPLIT_US us a layer where
+// Qwen2-7B heads (28 over 4) at 2000-2256 positions: 9.2 us a layer where
 // one position and head at a time on the VALU (a 64-lane sum for every score)
-// took 15.6, and the merge COMB_US us (6.7).  (Merging the ranges in the last
+// took 15.6, and the merge 4.4 us (6.7).  (Merging the ranges in the last
 // workgroup to finish, behind a device-scope counter, measured slower than the
 // separate merge kernel: the fences that make the partial sums visible across
 // the XCDs' L2 caches cost more than the launch.)
@@ -457,8 +457,13 @@ __global__ void __launch_bounds__(1024) attn_combine_k(const float *__restrict__
 // per wave there: a workgroup then loads the rows of about the positions it
 // has, 64 at a time, instead of 128 (decode +0.4 %).
 constexpr uint32_t kHeadWaves = 16;
-// cached positions up to which the forward pass uses attn_rope_head_k
-constexpr uint32_t kShortSeq = 512;
+// cached positions up to which the forward pass uses attn_rope_head_k, with two
+// ranges per head and with one.  Measured per layer against the split kernel
+// and its merge, whose time hardly depends on the length (us, whole step):
+// two ranges 56.8 / 58.7 at 500 positions and 59.0 / 58.6 at 700 (Qwen2-7B),
+// 55.0 / 55.7 and 57.3 / 55.7 (Llama-3-8B); one 28.5 / 29.9 at 200 and 32.1 /
+// 30.0 at 400 (Qwen2-0.5B).
+constexpr uint32_t kShortSeq = 512, kShortSeq1 = 256;
 template <int E, int NR = 1>
 __global__ void __launch_bounds__(64 * kHeadWaves) attn_rope_head_k(AttnArgs a, float *__restrict__ out)
 {
@@ -1296,16 +1301,17 @@ bool two_range_ok(const qg_model *m)
 }
 
 // the attention mode of the forward pass that writes cache slot `slot`: up to
-// kShortSeq cached positions whole heads, as two position ranges per head
-// where every wo takes them (mode 2) or in one workgroup per head (mode 1);
-// beyond, split over position ranges (mode 0).  att_path: 0 by length, 1
+// kShortSeq cached positions whole heads as two position ranges per head
+// where every wo takes them (mode 2), else up to kShortSeq1 in one workgroup
+// per head (mode 1); beyond, split over position ranges (mode 0).  att_path: 0 by length, 1
 // always one workgroup per head, 2 always split, 3 always two ranges where
 // the wo matrices allow it (else one workgroup per head).
 void pick_attention(qg_model *m, uint32_t slot)
 {
-    const bool shrt = m->att_path == 1 || m->att_path == 3 || (m->att_path == 0 && slot + 1 <= qgm::kShortSeq);
-    if (!m->att_grp || !shrt) m->att_mode = 0;
-    else m->att_mode = m->att_path != 1 && two_range_ok(m) ? 2 : 1;
+    const int whole = m->att_path != 1 && two_range_ok(m) ? 2 : 1;
+    const uint32_t most = whole == 2 ? qgm::kShortSeq : qgm::kShortSeq1;
+    const bool shrt = m->att_path == 1 || m->att_path == 3 || (m->att_path == 0 && slot + 1 <= most);
+    m->att_mode = m->att_grp && shrt ? whole : 0;
 }
 
 int run_forward(qg_model *m, uint32_t slot)

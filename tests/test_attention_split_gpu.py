@@ -1,0 +1,51 @@
+"""The split decode attention (attn_rope_split_k, attn_combine_k) against the
+oracle where its tiles and ranges end: 1 to 65 cached positions (a wave of 16
+with none, one and all of its positions, the second tile of 64), 4100 (ranges
+of two tiles), grouped heads of every size up to 8 and one, head_dim 64, 128
+and 256.  The prompt goes through the token-by-token path up to 70 positions,
+so every length is checked; DEEP_TOL (1e-4 normwise)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import normwise_err
+from test_decode_gpu import DEEP_TOL, SMALL, build
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("embed,heads,kv", [(256, 4, 2), (448, 7, 1), (512, 8, 1), (1024, 8, 8), (1024, 4, 1)])
+def test_every_length(rinf, synth, oracle, ctx, embed, heads, kv):
+    cfg = dict(SMALL, embed_dim=embed, n_heads=heads, n_kv_heads=kv, n_layers=1)
+    dev, ref, _ = build(rinf, synth, oracle, ctx, cfg, "q8_0", 31, 80)
+    dev.set_attention_path(2)
+    logits = np.zeros(cfg["vocab_size"], np.float32)
+    for pos in range(70):
+        tok = (pos * 37 + 5) % cfg["vocab_size"]
+        dev.forward(tok, pos, logits)
+        assert normwise_err(logits, ref.forward(tok, pos)) <= DEEP_TOL, pos
+    # a shorter conversation over the same cache: rows past it hold old values
+    dev.reset()
+    dev2, ref2, _ = build(rinf, synth, oracle, ctx, cfg, "q8_0", 31, 80)
+    dev2.close()
+    for pos in range(5):
+        tok = (pos * 91 + 1) % cfg["vocab_size"]
+        dev.forward(tok, pos, logits)
+        assert normwise_err(logits, ref2.forward(tok, pos)) <= DEEP_TOL, pos
+    dev.close()
+
+
+def test_ranges_of_two_tiles(rinf, synth, oracle, ctx):
+    cfg = dict(SMALL, embed_dim=128, n_heads=2, n_kv_heads=1, hidden_dim=128, n_layers=1, vocab_size=300)
+    n = 4100
+    dev, ref, _ = build(rinf, synth, oracle, ctx, cfg, "q8_0", 33, n + 40)
+    prompt = np.random.default_rng(5).integers(0, 300, n)
+    dev.prefill(prompt)
+    for pos, tok in enumerate(prompt):
+        ref.forward(int(tok), pos)
+    logits = np.zeros(300, np.float32)
+    for i in range(30):
+        dev.forward(i, n + i, logits)
+        assert normwise_err(logits, ref.forward(i, n + i)) <= DEEP_TOL, i
+    dev.close()
