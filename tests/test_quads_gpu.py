@@ -48,10 +48,12 @@ def test_ragged_rows(rinf, synth, oracle, ctx, t, rows, cols):
 
 
 @pytest.mark.parametrize("t", TYPES)
-@pytest.mark.parametrize("rows,cols", [(5, 32), (12, 96), (10, 896), (4099, 4096)])
+@pytest.mark.parametrize("rows,cols", [(5, 32), (12, 96), (10, 896), (3, 128), (9, 512), (17, 3840), (4099, 4096),
+                                       (5000, 256)])
 def test_f32_mode(rinf, synth, oracle, t, rows, cols):
-    """Both shapes of the kernel (a wave per row, four rows per workgroup), both
-    layouts, and the values themselves."""
+    """Every shape of the kernels (units of 32 elements, a wave per row, four rows
+    per workgroup), more rows than one round of workgroups, rows that start in
+    the middle of a block, and the values themselves."""
     c = rinf.GpuContext(0)
     c.set_precision(rinf.PRECISION_F32)
     dtype, raw = blocks(rinf, synth, t, rows, cols, rows + cols)
