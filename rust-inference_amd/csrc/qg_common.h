@@ -142,6 +142,8 @@ int launch_dequantize_row(uint32_t type, const uint8_t *w, size_t rows, size_t c
 int launch_dequantize_row_dev(uint32_t type, const uint8_t *w, size_t rows, size_t cols, const uint32_t *d_row,
                               float *out, ihipStream_t *stream);
 int launch_fill(float *out, size_t n, float v, ihipStream_t *stream);
+// dst = src, n floats, 16-byte aligned; either may be pinned host memory
+int launch_copy(float *dst, const float *src, size_t n, ihipStream_t *stream);
 // Batched prefill (qg_prefill.hip): tokens per chunk, supported matrix types,
 // and the launchers of its kernels (0 = launched, -1 = shape not supported,
 // -2 = launch failure).  x of every token t scaled per 256-element group g by

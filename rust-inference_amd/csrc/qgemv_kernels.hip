@@ -356,6 +356,14 @@ __device__ __forceinline__ float silu1(float x)
     return x * e / (1.0f + e);
 }
 
+// dst = src, 16-byte aligned both (one of them host memory: qg_matvec_host)
+__global__ void __launch_bounds__(256) copy_k(float *__restrict__ dst, const float *__restrict__ src, uint64_t n)
+{
+    const uint64_t i0 = (uint64_t)blockIdx.x * 256u + threadIdx.x, stride = (uint64_t)gridDim.x * 256u;
+    for (uint64_t i = i0; i < n / 4u; i += stride) *(f4 *)(dst + 4u * i) = *(const f4 *)(src + 4u * i);
+    if (i0 < (n & 3u)) dst[n - 1u - i0] = src[n - 1u - i0];
+}
+
 __global__ void fill_k(float *out, uint64_t n, float v)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -3352,6 +3360,15 @@ int launch_dequantize_rows_dev(uint32_t type, const uint8_t *w, size_t rows, siz
                                uint32_t n, float *out, size_t ldo, ihipStream_t *stream)
 {
     return launch_dequantize_row_any(type, w, rows, cols, 0, d_rows, n, out, ldo, stream);
+}
+
+int launch_copy(float *dst, const float *src, size_t n, ihipStream_t *stream)
+{
+    if (n == 0) return 0;
+    const size_t wgs = (n / 4u + 255u) / 256u;
+    hipLaunchKernelGGL(copy_k, dim3((unsigned)(wgs < 1u ? 1u : wgs < 256u ? wgs : 256u)), dim3(256), 0, (hipStream_t)stream,
+                       dst, src, (uint64_t)n);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
 int launch_fill(float *out, size_t n, float v, ihipStream_t *stream)
