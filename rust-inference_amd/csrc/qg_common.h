@@ -49,6 +49,7 @@ struct Plan {
     uint64_t group_bytes;  // bytes per row group
     uint32_t n_teams;      // teams in the grid
     uint32_t grid, block;  // launch shape
+    uint32_t cus;          // the device's compute units
     uint32_t R;            // row groups per batch
     uint32_t n_batches;    // ceil(n_groups / R)
     uint32_t per_team;     // batches each team runs

@@ -2730,6 +2730,7 @@ template <uint32_t T> static void plan_stream(size_t rows, size_t cols, int n_cu
     while (chunk > 1 && nw * chunk * red * 4u > room) chunk >>= 1;
     const uint32_t lds = img + (tsub == 0 ? nw * chunk * red * 4u : 0u);
     if (lds > (uint32_t)max_lds_bytes()) return;
+    p->cus = (uint32_t)ncu;
     p->fn = fn;
     p->fn_norm = fn_norm;
     p->fn_silu = fn_silu;
@@ -3085,16 +3086,26 @@ int launch_gemv_norm_glu(const Plan &p, const uint8_t *w, size_t nbytes, size_t 
 {
     // each half a whole number of row groups
     if (p.kind != 1 || !p.fn_norm_glu || p.tsub == 0 || rows % (2u * p.g) != 0 || cols % 4 != 0) return -1;
-    const uint32_t half = (uint32_t)(rows / 2 / p.g), tpw = p.block / p.ts;
-    const uint32_t pairs = (p.per_team + 1) / 2;
-    const uint32_t grid = (half + tpw * pairs - 1) / (tpw * pairs);
+    const uint32_t half = (uint32_t)(rows / 2 / p.g), pairs = (p.per_team + 1) / 2;
+    // The plan's workgroups hold one row group per team; a team takes two here
+    // (gate and up). Where that leaves one pair per team, smaller workgroups
+    // on as many CUs as there are, a thread's share of x still in registers
+    // (two 16-element pieces): Qwen2-0.5B's [gate; up], 122 workgroups of 320
+    // threads, 7.4 us, is 203 of 192, 5.6 us
+    uint32_t block = p.block;
+    for (uint32_t b = 64; pairs == 1 && b < p.block; b += 64)
+        if (b % p.ts == 0 && cols <= 32u * b && half <= p.cus * (b / p.ts)) {
+            block = b;
+            break;
+        }
+    const uint32_t tpw = block / p.ts, grid = (half + tpw * pairs - 1) / (tpw * pairs);
     StreamArgs a = stream_args(p, w, nbytes, rows, cols, xa, y);
     a.n_teams = grid * tpw;
     a.per_team = 2 * pairs;
     a.glu_half = half;
     a.xb = xb; a.nw = nw; a.sum_out = sum_out; a.eps = eps;
     void *args[] = {&a};
-    return hipLaunchKernel(p.fn_norm_glu, dim3(grid), dim3(p.block), args, p.lds, (hipStream_t)stream) ==
+    return hipLaunchKernel(p.fn_norm_glu, dim3(grid), dim3(block), args, p.lds, (hipStream_t)stream) ==
                    hipSuccess ? 0 : -2;
 }
 
@@ -3131,11 +3142,11 @@ static bool pair_part_ok(const Plan &p)
     return p.kind == 1 && p.tsub != 0 && kPairBlock % p.ts == 0;
 }
 
-// Workgroups of kPairBlock threads for a part of n_batches batches, per
-// batches per team.
-static uint32_t pair_grid(const Plan &p, uint32_t per)
+// Workgroups of `block` threads for a part of n_batches batches, per batches
+// per team.
+static uint32_t pair_grid(const Plan &p, uint32_t per, uint32_t block)
 {
-    const uint32_t tpw = kPairBlock / p.ts;
+    const uint32_t tpw = block / p.ts;
     return (p.n_batches + tpw * per - 1) / (tpw * per);
 }
 
@@ -3168,15 +3179,26 @@ int launch_gemv_norm_pair(uint32_t t1, const Plan &p1, const uint8_t *w1, size_t
     // per team for the part with more workgroups until they fit
     const uint64_t slots = (uint64_t)(n_cu > 0 ? n_cu : 256) * (uint64_t)pair_occupancy(fn, lds);
     uint32_t per1 = p1.per_team ? p1.per_team : 1u, per2 = p2.per_team ? p2.per_team : 1u;
-    uint32_t g1 = pair_grid(p1, per1), g2 = pair_grid(p2, per2);
+    // Small parts run in smaller workgroups, one team batch each, on as many
+    // CUs as there are, where a thread still holds its share of x in
+    // registers (two 16-element pieces): Qwen2-0.5B's [Q;K] and V, 18 + 4
+    // workgroups of 512 threads in 6.2 us, are 144 + 32 of 64 in 4.4
+    uint32_t block = kPairBlock;
+    for (uint32_t b : {64u, 128u, 256u})
+        if (per1 == 1u && per2 == 1u && b % p1.ts == 0 && b % p2.ts == 0 && cols <= 32u * b &&
+            (uint64_t)pair_grid(p1, 1u, b) + pair_grid(p2, 1u, b) <= (uint64_t)(n_cu > 0 ? n_cu : 256)) {
+            block = b;
+            break;
+        }
+    uint32_t g1 = pair_grid(p1, per1, block), g2 = pair_grid(p2, per2, block);
     while ((uint64_t)g1 + g2 > slots && (g1 > 1 || g2 > 1)) {
-        if (g1 >= g2) g1 = pair_grid(p1, ++per1);
-        else g2 = pair_grid(p2, ++per2);
+        if (g1 >= g2) g1 = pair_grid(p1, ++per1, block);
+        else g2 = pair_grid(p2, ++per2, block);
     }
     StreamArgs a1 = stream_args(p1, w1, nbytes1, rows1, cols, xa, y1);
     StreamArgs a2 = stream_args(p2, w2, nbytes2, rows2, cols, xa, y2);
-    a1.n_teams = g1 * (kPairBlock / p1.ts);
-    a2.n_teams = g2 * (kPairBlock / p2.ts);
+    a1.n_teams = g1 * (block / p1.ts);
+    a2.n_teams = g2 * (block / p2.ts);
     a1.per_team = per1;
     a2.per_team = per2;
     a1.xb = a2.xb = xb;
@@ -3184,7 +3206,7 @@ int launch_gemv_norm_pair(uint32_t t1, const Plan &p1, const uint8_t *w1, size_t
     a1.eps = a2.eps = eps;
     a1.sum_out = sum_out;
     void *args[] = {&a1, &a2, &g1};
-    return hipLaunchKernel(fn, dim3(g1 + g2), dim3(kPairBlock), args, lds, (hipStream_t)stream) == hipSuccess ? 0
+    return hipLaunchKernel(fn, dim3(g1 + g2), dim3(block), args, lds, (hipStream_t)stream) == hipSuccess ? 0
                                                                                                              : -2;
 }
 
