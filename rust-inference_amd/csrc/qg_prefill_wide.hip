@@ -656,8 +656,8 @@ __global__ void __launch_bounds__(512) wide_planes_k(const float *__restrict__ a
 // ------------------------------------------------------------- attention
 
 // Causal attention of query head blockIdx.x for the chunk's tokens t0 .. t0 +
-// 63 (the last token tiles first: they see the most positions), token t over
-// cache slots 0 .. slot0 + t (attention.rs:93-121, math.rs:63-70 / 104-118).
+// 63, token t over cache slots 0 .. slot0 + t (attention.rs:93-121,
+// math.rs:63-70 / 104-118).
 // Four waves of 16 tokens; positions in tiles of 32 rows of K and V, staged in
 // LDS for the four and requested one tile ahead.  A wave computes S = Q K^T
 // (2 x hd / 4 v_mfma_f32_16x16x4f32, Q in registers), its running maximum per
@@ -707,7 +707,13 @@ __global__ void __launch_bounds__(256) wide_attention_k(const float *__restrict_
     const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, g = lane >> 4;
     const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
     float *ps = vs + kAttPos * LK + w * 16u * LP;
-    const uint32_t h = blockIdx.x, t0 = (gridDim.y - 1u - blockIdx.y) * kAttTok, kvh = (h / n_rep) * HD;
+    // token tiles: the later half from the last on, then the earlier half from
+    // the first on, so that a CU's second workgroup is the shorter the longer
+    // its first (1001 tokens of 32 heads: 130 us; all from the last on 139;
+    // eight waves, four of them for the second half of tiles of 64 positions,
+    // 154)
+    const uint32_t ny = gridDim.y, by = blockIdx.y, late = (ny + 1u) / 2u;
+    const uint32_t h = blockIdx.x, t0 = (by < late ? ny - 1u - by : by - late) * kAttTok, kvh = (h / n_rep) * HD;
     const uint32_t tw = t0 + 16u * w;                      // this wave's first token
     const uint32_t npos = slot0 + min(ntok, t0 + kAttTok); // positions any token of the workgroup sees
     // A of S: q[token c][16 k + 4 g + j] (tokens past the chunk: the last one's, never stored)
