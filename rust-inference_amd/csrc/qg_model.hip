@@ -1559,13 +1559,23 @@ int wide_alloc(qg_model *m)
         rg = std::max(rg, t * s.gu);
         rd = std::max(rd, t * s.down);
     }
+    const size_t held = m->allocs.size(), bytes = m->alloc_bytes;
     int rc;
-    if ((!m->wd_h[0] && (rc = dalloc(m, &m->wd_h[0], T * E))) || (!m->wd_h[1] && (rc = dalloc(m, &m->wd_h[1], T * E))) ||
-        (!m->wd_qkv && (rc = dalloc(m, &m->wd_qkv, rq * ldq))) || (!m->wd_ao && (rc = dalloc(m, &m->wd_ao, T * m->q_dim))) ||
-        (!m->wd_ao2 && (rc = dalloc(m, &m->wd_ao2, ro * E))) || (!m->wd_g && (rc = dalloc(m, &m->wd_g, rg * 2 * H))) ||
-        (!m->wd_fo && (rc = dalloc(m, &m->wd_fo, rd * E))) || (!m->wd_xp && (rc = dalloc(m, &m->wd_xp, T * kmax * 4))) ||
-        (!m->wd_rec && (rc = dalloc(m, &m->wd_rec, T * kmax / 32))) || (!m->wd_scl && (rc = dalloc(m, &m->wd_scl, T))))
+    if (qg_alloc_injected(m->ctx)) rc = mfail(m, QG_ERR_OUT_OF_MEMORY, "hipMalloc (injected failure)");
+    else if ((rc = dalloc(m, &m->wd_h[0], T * E)) || (rc = dalloc(m, &m->wd_h[1], T * E)) ||
+             (rc = dalloc(m, &m->wd_qkv, rq * ldq)) || (rc = dalloc(m, &m->wd_ao, T * m->q_dim)) ||
+             (rc = dalloc(m, &m->wd_ao2, ro * E)) || (rc = dalloc(m, &m->wd_g, rg * 2 * H)) ||
+             (rc = dalloc(m, &m->wd_fo, rd * E)) || (rc = dalloc(m, &m->wd_xp, T * kmax * 4)) ||
+             (rc = dalloc(m, &m->wd_rec, T * kmax / 32)))
+        ;
+    else rc = dalloc(m, &m->wd_scl, T);
+    if (rc) {                                            // all of them or none
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(m->ctx->stream);
+        for (; m->allocs.size() > held; m->allocs.pop_back()) (void)hipFree(m->allocs.back());
+        m->alloc_bytes = bytes;
         return rc;
+    }
     m->pf_wide = cap;
     return QG_OK;
 }
@@ -1661,9 +1671,13 @@ int prefill(qg_model *m, const uint32_t *tok, size_t n)
         QGM_HIP(m, hipMemcpyAsync(m->pf_tok, tok, n * sizeof(uint32_t), hipMemcpyHostToDevice, m->ctx->stream));
         QGM_HIP(m, hipStreamSynchronize(m->ctx->stream));
         // more than one narrow chunk's tokens: wide chunks of equal length (in
-        // whole tiles), where every matrix takes them
-        const bool wide = n > qg::kPfMaxTokens && wide_supported(m);
-        if (wide && (rc = wide_alloc(m))) return rc;
+        // whole tiles), where every matrix takes them and the card has room
+        // for their buffers
+        bool wide = n > qg::kPfMaxTokens && wide_supported(m);
+        if (wide && (rc = wide_alloc(m))) {
+            if (rc != QG_ERR_OUT_OF_MEMORY) return rc;
+            wide = false;
+        }
         size_t len = qg::kPfMaxTokens;
         if (wide) {
             const size_t parts = (n + m->pf_wide - 1) / m->pf_wide, per = (n + parts - 1) / parts;

@@ -8,9 +8,11 @@ greedy steps after the prompt read every cached position.  Tolerance: DEEP_TOL
 (1e-4 normwise, the bound of the decode and prefill tests)."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 
-from test_decode_gpu import DEEP_TOL, SMALL
+from conftest import normwise_err
+from test_decode_gpu import DEEP_TOL, SMALL, build
 from test_prefill_gpu import prefill_and_compare
 
 pytestmark = pytest.mark.gpu
@@ -38,3 +40,24 @@ def test_two_chunks_and_continued(rinf, synth, oracle, ctx):
     e0, errs, _ = prefill_and_compare(rinf, synth, oracle, ctx, SMALL, "q4_k_m", 7, 1100, 3, 1200)
     e1, errs1, _ = prefill_and_compare(rinf, synth, oracle, ctx, SMALL, "q5_k_m", 8, 300, 3, 400, split=81)
     assert max([e0, e1] + errs + errs1) <= DEEP_TOL, (e0, errs, e1, errs1)
+
+
+def test_no_room_for_the_wide_buffers(rinf, synth, oracle, ctx):
+    """Where the wide chunks' buffers cannot be allocated the prompt goes through
+    64-token chunks; the next prompt finds room and takes the wide ones."""
+    dev, ref, shared = build(rinf, synth, oracle, ctx, SMALL, "q4_k_m", 11, 400)
+    prompt = np.random.default_rng(11).integers(0, SMALL["vocab_size"], 330)
+    logits = np.zeros(SMALL["vocab_size"], np.float32)
+    pos = 0
+    for part, fail in ((prompt[:40], False), (prompt[40:190], True), (prompt[190:], False)):
+        if fail:
+            ctx.fail_allocations(1)
+        dev.prefill(part, logits)
+        ctx.fail_allocations(0)
+        for tok in part:
+            ref_l = ref.forward(int(tok), pos)
+            pos += 1
+        assert normwise_err(logits, ref_l) <= DEEP_TOL, pos
+    dev.close()
+    if shared is not None:
+        shared.free()
