@@ -418,7 +418,7 @@ def shape_run(rinf, synth, ctx, torch, tname, rows, cols, steps, warmup, rotate_
     c_ms, eager_ms, graph_ms, _ = time_gemv(ctx, torch, mats, dx, dy, steps, warmup)
     us = min(c_ms, eager_ms, graph_ms) * 1e3 / steps
     B = alg_bytes(rinf, dtype, rows, cols)
-    kind = {1: "gemv_stream", 2: "gemv_ring", 3: "gemv_wave"}.get(mats[0].kernel_kind, "gemv_generic")
+    kind = {1: "gemv_stream", 2: "gemv_ring", 3: "gemv_wave"}.get(mats[0].kernel_kind, "gemv_quads")
     if not np.all(np.isfinite(dy.cpu().numpy())):
         raise SystemExit(f"{tname} {rows}x{cols}: non-finite output")
     for m in mats:
@@ -712,7 +712,7 @@ def main():
     raw = synth.gen_blocks(dtype, rows, cols, synth.config_seed(4))
     x = synth.gen_x(cols, synth.config_seed(4))
     mats = [ctx.upload(raw, dtype, rows, cols) for _ in range(ncopy)]
-    kernel = {1: "qg::gemv_stream", 2: "qg::gemv_ring", 3: "qg::gemv_wave"}.get(mats[0].kernel_kind, "qg::gemv_generic")
+    kernel = {1: "qg::gemv_stream", 2: "qg::gemv_ring", 3: "qg::gemv_wave"}.get(mats[0].kernel_kind, "qg::gemv_quads")
     dx = torch.from_numpy(x).cuda()
     dy = torch.zeros(rows, dtype=torch.float32, device="cuda")
     torch.cuda.synchronize()
