@@ -91,10 +91,9 @@ int qg_model_forward(qg_model *m, uint32_t token, uint32_t pos, float *logits);
  * qg_model_forward would -- the logits are the last token's.  Chunks of up to
  * 64 tokens (prompts of more than 64: up to 1024) go through each layer
  * together, every projection one f16 MFMA GEMM over the tokens' x split into
- * two f16 pieces under a power-of-two scale per 256 elements (chunks of more
- * than 64 tokens: per token; batched prefill, exact products, f32
- * accumulation) and the attention on f32 MFMAs, when every layer matrix is
- * Q4_K, Q5_K, Q6_K or Q8_0 with cols % 128 == 0 and head_dim is 64, 128 or
+ * two f16 pieces under a power-of-two scale per 256 elements (batched prefill,
+ * exact products, f32 accumulation) and the attention on f32 MFMAs, when every
+ * layer matrix is Q4_K, Q5_K, Q6_K or Q8_0 with cols % 128 == 0 and head_dim is 64, 128 or
  * 256; otherwise, or after qg_model_use_batched_prefill(m, 0), one forward
  * pass per token.  `logits`,
  * if not NULL, receives vocab_size floats (host memory).  QG_ERR_SHAPE when

@@ -204,11 +204,11 @@ int launch_pf_attention(const float *qkv, uint32_t ldq, const float *kc, const f
                         ihipStream_t *stream);
 // Prefill of more than kPfMaxTokens tokens (qg_prefill_wide.hip): up to
 // kWideMax tokens per launch, repacked matrices of at most kWideCols columns,
-// at most kWideSlices K slices.  x of every token scaled by one power of two
-// 2^e, as two f16 pieces: per 64 tokens and 128-element chunk a 32 KB image in
-// xp, the sums of xs per 32 elements (two f16 pieces, [chunk][4][64 tokens]) in
-// rec, 2^-e per token in scl; tokens in whole tiles of 128 (xp 4 n, rec n / 8
-// and scl 4 bytes per token of the tiles).
+// at most kWideSlices K slices.  x of every token scaled per 256-element group g
+// by a power of two 2^e_g, as two f16 pieces: per 64 tokens and 128-element
+// chunk a 32 KB image in xp, and in rec five rows of 64 tokens: the sums of xs
+// of the chunk's four 32-element segments (two f16 pieces), 2^-e_g; tokens in
+// whole tiles of 128 (xp 4 n, rec 5 n / 32 bytes per token of the tiles).
 constexpr uint32_t kWideMax = 1024, kWideCols = 32768, kWideSlices = 8, kWideTile = 128;
 bool wide_mat_ok(const PfMat &m, size_t cols);
 uint32_t wide_tiles(size_t rows);
@@ -217,13 +217,12 @@ uint32_t wide_split(uint32_t row_tiles, uint32_t tok_tiles, size_t cols);
 // 1..3 matrices of one type (and all or none with one row per group) over the
 // same x; slice s of a result at y + s * sstride, y[t * ldy + r]
 int launch_wide_gemm(const PfMat *mats, int n_mats, size_t cols, const uint8_t *xp, const uint32_t *rec,
-                     const float *scl, uint32_t ntok, uint32_t ldy, uint32_t slices, size_t sstride,
-                     ihipStream_t *stream);
+                     uint32_t ntok, uint32_t ldy, uint32_t slices, size_t sstride, ihipStream_t *stream);
 // x = f(a, b) (sums of na / nb slices; rows of lda floats): mode 0: a; 1:
 // rmsnorm(a + b) * nw, sum_out (may be NULL) = a + b; 2: silu(a) * b
 int launch_wide_planes(const float *a, uint32_t na, const float *b, uint32_t nb, size_t sstride, float *sum_out,
                        const float *nw, size_t n, size_t lda, int mode, float eps, uint8_t *xp, uint32_t *rec,
-                       float *scl, uint32_t ntok, ihipStream_t *stream);
+                       uint32_t ntok, ihipStream_t *stream);
 int launch_wide_attention(const float *qkv, uint32_t ldq, const float *kc, const float *vc, float *out,
                           uint32_t n_heads, uint32_t hd, uint32_t kv_dim, uint32_t n_rep, float scale, uint32_t slot0,
                           uint32_t ntok, ihipStream_t *stream);

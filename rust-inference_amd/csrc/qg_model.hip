@@ -842,7 +842,7 @@ struct qg_model {
     // pf_wide tokens per chunk: the same buffers for whole tiles of tokens
     uint32_t pf_wide = 0;
     float *wd_h[2] = {nullptr, nullptr}, *wd_qkv = nullptr, *wd_ao = nullptr, *wd_ao2 = nullptr, *wd_g = nullptr,
-          *wd_fo = nullptr, *wd_scl = nullptr;
+          *wd_fo = nullptr;
     uint8_t *wd_xp = nullptr;
     uint32_t *wd_rec = nullptr;
     // captured graphs per attention mode: [0] the split attention
@@ -1565,10 +1565,9 @@ int wide_alloc(qg_model *m)
     else if ((rc = dalloc(m, &m->wd_h[0], T * E)) || (rc = dalloc(m, &m->wd_h[1], T * E)) ||
              (rc = dalloc(m, &m->wd_qkv, rq * ldq)) || (rc = dalloc(m, &m->wd_ao, T * m->q_dim)) ||
              (rc = dalloc(m, &m->wd_ao2, ro * E)) || (rc = dalloc(m, &m->wd_g, rg * 2 * H)) ||
-             (rc = dalloc(m, &m->wd_fo, rd * E)) || (rc = dalloc(m, &m->wd_xp, T * kmax * 4)) ||
-             (rc = dalloc(m, &m->wd_rec, T * kmax / 32)))
+             (rc = dalloc(m, &m->wd_fo, rd * E)) || (rc = dalloc(m, &m->wd_xp, T * kmax * 4)))
         ;
-    else rc = dalloc(m, &m->wd_scl, T);
+    else rc = dalloc(m, &m->wd_rec, T * kmax / 128 * 5);
     if (rc) {                                            // all of them or none
         (void)hipGetLastError();
         (void)hipStreamSynchronize(m->ctx->stream);
@@ -1587,7 +1586,7 @@ int wide_gemm(qg_model *m, const qg::PfMat *mats, int n, size_t cols, uint32_t n
     for (int i = 0; i < n;) {
         int k = i + 1;
         while (k < n && mats[k].type == mats[i].type && (mats[k].g == 1) == (mats[i].g == 1)) k++;
-        if (qg::launch_wide_gemm(mats + i, k - i, cols, m->wd_xp, m->wd_rec, m->wd_scl, ntok, ldy, slices, sstride,
+        if (qg::launch_wide_gemm(mats + i, k - i, cols, m->wd_xp, m->wd_rec, ntok, ldy, slices, sstride,
                                  (ihipStream_t *)m->ctx->stream))
             return mfail(m, QG_ERR_HIP, "prefill GEMM launch", hipGetLastError());
         i = k;
@@ -1599,7 +1598,7 @@ int wide_planes(qg_model *m, const float *a, uint32_t na, const float *b, uint32
                 const float *nw, size_t n, size_t lda, int mode, uint32_t ntok)
 {
     if (qg::launch_wide_planes(a, na, b, nb, sstride, sum_out, nw, n, lda, mode, m->cfg.norm_eps, m->wd_xp, m->wd_rec,
-                               m->wd_scl, ntok, (ihipStream_t *)m->ctx->stream))
+                               ntok, (ihipStream_t *)m->ctx->stream))
         return mfail(m, QG_ERR_HIP, "prefill planes launch", hipGetLastError());
     return QG_OK;
 }

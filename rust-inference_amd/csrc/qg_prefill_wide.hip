@@ -7,15 +7,16 @@
 //
 //   * wide_planes_k: one workgroup per token holds the token's whole input
 //     vector x (the RMSNorm of the residual stream, the attention output, or
-//     silu(g) * u), so x has ONE power-of-two scale 2^e per token (its largest
-//     magnitude into [512, 1024)) and the norm is complete; xs = x 2^e goes out
-//     as two f16 pieces (hi + lo, 22 significant bits of everything down to
-//     2^-12 of the token's maximum, and an absolute 2^-35 of it below) in the
-//     layout of the GEMM's LDS buffers, with the sums of xs per 32 elements;
+//     silu(g) * u), so the norm is complete; every 256-element group g of x has
+//     its own power-of-two scale 2^e_g (the group's largest magnitude into
+//     [512, 1024)), as in qg_prefill.hip, and xs = x 2^e_g goes out as two f16
+//     pieces (hi + lo, 22 significant bits of everything down to 2^-12 of the
+//     group's maximum, and an absolute 2^-35 of it below) in the layout of the
+//     GEMM's LDS buffers, with the sums of xs per 32 elements and 2^-e_g;
 //   * wide_gemm_k: tiles of 128 tokens x 256 rows,
-//     y = 2^-e (sum over blocks of d D - dmin Dm): D the block's exact integer
-//     products accumulated by v_mfma_f32_16x16x32_f16, Dm its min terms by
-//     v_mfma_f32_16x16x16_f16;
+//     y = sum over blocks of 2^-e_g (d D - dmin Dm): D the block's exact
+//     integer products accumulated by v_mfma_f32_16x16x32_f16, Dm its min terms
+//     by v_mfma_f32_16x16x16_f16;
 //   * wide_attention_k: causal attention, 64 tokens of a head per workgroup,
 //     on v_mfma_f32_16x16x4f32 (f32 products and sums).
 //
@@ -247,8 +248,10 @@ constexpr uint32_t kTok = 128;                     // tokens per workgroup tile:
 constexpr uint32_t kRowsWG = 8u * 16u * kR;        // rows per workgroup tile
 constexpr uint32_t kImg = 2u * 64u * 256u;         // bytes of a chunk's x image of 64 tokens
 constexpr uint32_t kBufX = 2u * kImg;              // ... of a workgroup's two halves
-constexpr uint32_t kBufS = 2u * 4u * 64u * 4u;     // bytes of a chunk's sums
-constexpr uint32_t kLds = 2u * kBufX + 4u * kBufS; // two x buffers, four of the sums
+// A chunk's record of 64 tokens: the sums of its four sub-blocks, then 2^-e_g
+constexpr uint32_t kRec = 5u * 64u;                // dwords
+constexpr uint32_t kBufS = 2u * kRec * 4u;         // bytes of a workgroup's two halves
+constexpr uint32_t kLds = 2u * kBufX + 4u * kBufS; // two x buffers, four of the records
 
 __device__ __forceinline__ void dma16(const void *gp, uint32_t lds_addr)
 {
@@ -299,18 +302,21 @@ struct Jobs {
 // queue fills and the waves wait to issue).  64-token chunks through
 // qg_prefill.hip's kernel, 16 of them: 1120 / 800.
 //
-// A token scale common to the row leaves one FMA per block and element for d D
-// and one for -dmin Dm.  ONE: one row per row group (blocks end with every
-// second chunk for the whole wave); otherwise rows may start in the middle of
-// a block and every chunk ends D.
+// ONE: one row per row group (blocks end with every second chunk for the whole
+// wave, and a block is a group of x); otherwise rows may start in the middle of
+// a block and every chunk ends D.  At the end of D the token's 2^-e_g comes
+// from the record, one multiply per element more than a scale common to the
+// row would take: nothing to see of it in the time (1001 tokens of two
+// Llama-3-8B layers, Q5_K and Q6_K: 2.73 ms with the common scale, 2.70 so),
+// and without it an outlier takes the bits of the whole row.
 //
 // Blocks go to XCDs so that the token tiles of a row tile run beside each
 // other on one XCD: its L2 then holds the row tile's open weight lines.
 template <uint32_t T, bool ONE>
 __global__ void __launch_bounds__(512) wide_gemm_k(Jobs jobs, uint32_t row_tiles, uint32_t tok_tiles, uint32_t slices,
                                                    uint32_t nchunk, uint32_t cps, const uint8_t *__restrict__ xp,
-                                                   const uint32_t *__restrict__ rec, const float *__restrict__ scl,
-                                                   uint32_t ntok, uint32_t ldy, uint64_t sstride)
+                                                   const uint32_t *__restrict__ rec, uint32_t ntok, uint32_t ldy,
+                                                   uint64_t sstride)
 {
     using P = Wt<T>;
     constexpr bool Q8 = T == T_Q8_0;
@@ -346,7 +352,7 @@ __global__ void __launch_bounds__(512) wide_gemm_k(Jobs jobs, uint32_t row_tiles
     // part `part` (of 4) of the copies of chunk c into buffer c' & 1 (c' = c, or
     // the chunk after the slice's last, whose buffers no one reads): wave w
     // copies 1 KB blocks 8 w .. 8 w + 7 of the chunk's 64 KB and the sums of one
-    // sub-block of a half
+    // sub-block of a half; waves 0 and 4 the halves' scales
     auto stage = [&](uint32_t c, uint32_t cd, uint32_t part) {
         const uint32_t b0 = lds0 + (cd & 1u) * kBufX;
         const size_t img = (size_t)(tg0 + (wave >> 2)) * nchunk + c;
@@ -354,8 +360,12 @@ __global__ void __launch_bounds__(512) wide_gemm_k(Jobs jobs, uint32_t row_tiles
 #pragma unroll
         for (uint32_t v = 2u * part; v < 2u * part + 2u; v++)
             dma16(src + v * 1024u + 16u * lane, b0 + wave * 8192u + v * 1024u);
-        if (part == 0u && P::KQ)
-            dma4(rec + img * 256u + (wave & 3u) * 64u + lane, lds0 + 2u * kBufX + (cd & 3u) * kBufS + wave * 256u);
+        if (part == 0u) {
+            const uint32_t *r = rec + img * kRec + lane;
+            const uint32_t rl = lds0 + 2u * kBufX + (cd & 3u) * kBufS + (wave >> 2) * 4u * kRec;
+            if (P::KQ) dma4(r + (wave & 3u) * 64u, rl + (wave & 3u) * 256u);
+            if ((wave & 3u) == 0u) dma4(r + 256u, rl + 1024u);
+        }
     };
     typename P::Raw cw[kR], nw[kR];
     v4u nh[kR];                                                   // K-quants: the next block's headers
@@ -425,10 +435,28 @@ __global__ void __launch_bounds__(512) wide_gemm_k(Jobs jobs, uint32_t row_tiles
                     }
                     P::decode(cw[i], sc[i], m, kq, b[i]);
                 }
-                const bool first = Q8 || (hc == 0 && m == 0);       // D starts at zero
+                const bool first = hc == 0 && m == 0;               // D starts at zero
 #pragma unroll
                 for (uint32_t t = 0; t < 8; t++) {
                     const h8 a0 = *(const h8 *)(xa + (t & 3u) * 4096u + (t >> 2) * 32768u), a1 = *(const h8 *)(xa + (t & 3u) * 4096u + (t >> 2) * 32768u + 16384u);
+                    if constexpr (Q8) {                             // a block per step: d times its products
+                        v4f q[kR];
+#pragma unroll
+                        for (uint32_t i = 0; i < kR; i++)
+                            q[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, __builtin_bit_cast(h8, b[i][0]),
+                                                                          v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                        for (uint32_t i = 0; i < kR; i++)
+                            q[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, __builtin_bit_cast(h8, b[i][0]), q[i], 0, 0, 0);
+#pragma unroll
+                        for (uint32_t i = 0; i < kR; i++) {
+                            const float d = Wt<T_Q8_0>::dscale(cw[i], m);
+#pragma unroll
+                            for (int e = 0; e < 4; e++)
+                                D[i][t][e] = first ? d * q[i][e] : __builtin_fmaf(d, q[i][e], D[i][t][e]);
+                        }
+                        continue;
+                    }
 #pragma unroll
                     for (uint32_t i = 0; i < kR; i++)
                         D[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, __builtin_bit_cast(h8, b[i][0]),
@@ -440,52 +468,49 @@ __global__ void __launch_bounds__(512) wide_gemm_k(Jobs jobs, uint32_t row_tiles
 #pragma unroll
                         for (uint32_t i = 0; i < kR; i++)
                             D[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, __builtin_bit_cast(h8, b[i][1]), D[i][t], 0, 0, 0);
-                    if constexpr (Q8) {                             // a scale per step
-#pragma unroll
-                        for (uint32_t i = 0; i < kR; i++) {
-                            const float d = Wt<T_Q8_0>::dscale(cw[i], m);
-#pragma unroll
-                            for (int e = 0; e < 4; e++) acc[i][t][e] = __builtin_fmaf(d, D[i][t][e], acc[i][t][e]);
-                        }
-                    }
                 }
             }
-            if constexpr (!Q8) {
-                if (hc + 1u == BLK) {
-                    // the end of D: d D, and the min terms -dmin Dm
-                    const uint8_t *sb = lds + 2u * kBufX + 4u * c16;
+            if (hc + 1u == BLK) {
+                // the end of D: acc += 2^-e_g (d D - dmin Dm), Dm the min terms
+                const uint8_t *sb = lds + 2u * kBufX;
+                float d[kR], dm[kR];
+                uint2 bm[kR];
+#pragma unroll
+                for (uint32_t i = 0; i < kR; i++) {
+                    if constexpr (P::KQ) {
+                        d[i] = h2f(hd[i].dd);
+                        dm[i] = -h2f(hd[i].dd >> 16);
+                        bm[i] = kmins(hd[i].m4, kq);
+                        if (BLK == 1u && kq >= 2u) bm[i] = make_uint2(0u, 0u);
+                    } else if constexpr (!Q8) {
+                        d[i] = h2f(cw[i].d);
+                    }
+                }
+#pragma unroll
+                for (uint32_t t = 0; t < 8; t++) {
+                    const uint32_t to = (t & 3u) * 64u + (t >> 2) * 4u * kRec;
+                    const v4f sg = *(const v4f *)(sb + (c & 3u) * kBufS + 1024u + to + 16u * kq);
+                    h4 sa = {};
+                    if constexpr (P::KQ) {
+                        // lane kq: the sums of sub-blocks 2 kq, 2 kq + 1 of the block (kq >> 1: its
+                        // chunk), or of the chunk's 2 (kq & 1), + 1
+                        const uint32_t cs = BLK == 2u ? cb + (kq >> 1) : c;
+                        const uint8_t *s = sb + (cs & 3u) * kBufS + (kq & 1u) * 512u + to + 4u * c16;
+                        sa = __builtin_bit_cast(h4, make_uint2(*(const uint32_t *)s, *(const uint32_t *)(s + 256u)));
+                    }
 #pragma unroll
                     for (uint32_t i = 0; i < kR; i++) {
-                        float d;
-                        if constexpr (P::KQ) d = h2f(hd[i].dd);
-                        else d = h2f(cw[i].d);
+                        if constexpr (P::KQ) {
+                            const v4f Dm = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, __builtin_bit_cast(h4, bm[i]),
+                                                                                 v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-                        for (uint32_t t = 0; t < 8; t++)
+                            for (int e = 0; e < 4; e++)
+                                acc[i][t][e] = __builtin_fmaf(sg[e], __builtin_fmaf(d[i], D[i][t][e], dm[i] * Dm[e]),
+                                                              acc[i][t][e]);
+                        } else {
 #pragma unroll
-                            for (int e = 0; e < 4; e++) acc[i][t][e] = __builtin_fmaf(d, D[i][t][e], acc[i][t][e]);
-                    }
-                    if constexpr (P::KQ) {
-                        h4 sa[8];
-#pragma unroll
-                        for (uint32_t t = 0; t < 8; t++) {
-                            // lane kq: the sums of sub-blocks 2 kq, 2 kq + 1 of the block (kq >> 1: its
-                            // chunk), or of the chunk's 2 (kq & 1), + 1
-                            const uint32_t cs = BLK == 2u ? cb + (kq >> 1) : c;
-                            const uint8_t *s = sb + (cs & 3u) * kBufS + (kq & 1u) * 512u + (t & 3u) * 64u + (t >> 2) * 1024u;
-                            sa[t] = __builtin_bit_cast(h4, make_uint2(*(const uint32_t *)s, *(const uint32_t *)(s + 256u)));
-                        }
-#pragma unroll
-                        for (uint32_t i = 0; i < kR; i++) {
-                            uint2 bm = kmins(hd[i].m4, kq);
-                            if (BLK == 1u && kq >= 2u) bm = make_uint2(0u, 0u);
-                            const float dm = -h2f(hd[i].dd >> 16);
-#pragma unroll
-                            for (uint32_t t = 0; t < 8; t++) {
-                                const v4f Dm = __builtin_amdgcn_mfma_f32_16x16x16f16(sa[t], __builtin_bit_cast(h4, bm),
-                                                                                     v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-                                for (int e = 0; e < 4; e++) acc[i][t][e] = __builtin_fmaf(dm, Dm[e], acc[i][t][e]);
-                            }
+                            for (int e = 0; e < 4; e++)
+                                acc[i][t][e] = __builtin_fmaf(Q8 ? sg[e] : d[i] * sg[e], D[i][t][e], acc[i][t][e]);
                         }
                     }
                 }
@@ -500,12 +525,11 @@ __global__ void __launch_bounds__(512) wide_gemm_k(Jobs jobs, uint32_t row_tiles
 #pragma unroll
         for (uint32_t e = 0; e < 4; e++) {
             const uint32_t tok = tb + 16u * t + 4u * kq + e;
-            const float s = scl[min(tok, ntok - 1u)];                               // 2^-e of the token, NaN if its x is not finite
             if (tok < ntok)
 #pragma unroll
                 for (uint32_t i = 0; i < kR; i++) {
                     const uint32_t r = row0 + 16u * i + c16;
-                    if (r < J.rows) y[(size_t)tok * ldy + r] = acc[i][t][e] * s;
+                    if (r < J.rows) y[(size_t)tok * ldy + r] = acc[i][t][e];
                 }
         }
 }
@@ -513,19 +537,15 @@ __global__ void __launch_bounds__(512) wide_gemm_k(Jobs jobs, uint32_t row_tiles
 // ---------------------------------------------------------------- planes
 
 // sum of v over a workgroup of 512 threads (every thread the same value); red: 8 floats
-template <bool MAX> __device__ __forceinline__ float block_red(float v, float *red)
+__device__ __forceinline__ float block_sum(float v, float *red)
 {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float u = __shfl_xor(v, o, 64);
-        v = MAX ? fmaxf(v, u) : v + u;
-    }
-    __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     float r = red[0];
 #pragma unroll
-    for (int i = 1; i < 8; i++) r = MAX ? fmaxf(r, red[i]) : r + red[i];
+    for (int i = 1; i < 8; i++) r += red[i];
     return r;
 }
 
@@ -551,17 +571,18 @@ __device__ __forceinline__ void sum8(const float *p, uint32_t ns, uint64_t sstri
 
 // The input vector x of token blockIdx.x -- mode 0: a; mode 1: rmsnorm(a + b)
 // * nw, with a + b stored to sum_out when given; mode 2: silu(a) * b -- as the
-// GEMM's x images: xs = x 2^e (the token's largest magnitude into [512, 1024))
-// in two f16 pieces, slot j (8 elements) of a chunk at position j ^ (t & 15)
-// of the token's 256 bytes, the sums of xs per 32 elements (two f16 pieces)
-// and 2^-e (NaN when the token's x is not finite).  a, b: sums of na, nb
-// slices.  PM: 8-element pieces per thread (n <= 4096 PM).
+// GEMM's x images: xs = x 2^e_g (the largest magnitude of the 256-element group
+// g into [512, 1024)) in two f16 pieces, slot j (8 elements) of a chunk at
+// position j ^ (t & 15) of the token's 256 bytes, the sums of xs per 32
+// elements (two f16 pieces) and 2^-e_g (NaN when the group's x is not finite),
+// of each of the group's chunks.  32 threads hold a group.  a, b: sums of na,
+// nb slices.  PM: 8-element pieces per thread (n <= 4096 PM).
 template <int PM>
 __global__ void __launch_bounds__(512) wide_planes_k(const float *__restrict__ a, uint32_t na, const float *__restrict__ b,
                                                      uint32_t nb, uint64_t sstride, float *__restrict__ sum_out,
                                                      const float *__restrict__ nw, uint32_t n, uint32_t lda,
                                                      uint32_t mode, float eps, uint8_t *__restrict__ xp,
-                                                     uint32_t *__restrict__ rec, float *__restrict__ scl)
+                                                     uint32_t *__restrict__ rec)
 {
     __shared__ float red[8];
     const uint32_t t = blockIdx.x, tid = threadIdx.x, np = n / 8u, nchunk = n / 128u;
@@ -593,7 +614,7 @@ __global__ void __launch_bounds__(512) wide_planes_k(const float *__restrict__ a
     }
     if (mode == 1u) {
         // math.rs:237-257: x * (1 / rms) * w
-        const float r = 1.0f / sqrtf(block_red<false>(ss, red) / (float)n + eps);
+        const float r = 1.0f / sqrtf(block_sum(ss, red) / (float)n + eps);
 #pragma unroll
         for (int p = 0; p < PM; p++) {
             const uint32_t j = tid + 512u * (uint32_t)p;
@@ -605,29 +626,28 @@ __global__ void __launch_bounds__(512) wide_planes_k(const float *__restrict__ a
             }
         }
     }
-    float mx = 0.f;
-    bool bad = false;
+    uint8_t *xt = xp + (size_t)(t >> 6) * nchunk * kImg + (t & 63u) * 256u;
+    uint32_t *rt = rec + (size_t)(t >> 6) * nchunk * kRec + (t & 63u);
 #pragma unroll
-    for (int p = 0; p < PM; p++)
+    for (int p = 0; p < PM; p++) {
+        const uint32_t j = tid + 512u * (uint32_t)p;
+        const bool live = j < np;
+        float mx = 0.f;
+        bool bad = false;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             bad |= !__builtin_isfinite(v[p][e]);
             mx = fmaxf(mx, fabsf(v[p][e]));
         }
-    // a NaN passes fmaxf by: it goes through the maximum as an infinity
-    mx = block_red<true>(bad ? INFINITY : mx, red);
-    bad = !__builtin_isfinite(mx);
-    int E = 0;
-    (void)frexpf(mx, &E);
-    const int e2 = bad || mx == 0.f ? 0 : min(max(10 - E, -126), 126);
-    const float sc = ldexpf(1.0f, e2);
-    if (tid == 0) scl[t] = bad ? __builtin_nanf("") : ldexpf(1.0f, -e2);
-    uint8_t *xt = xp + (size_t)(t >> 6) * nchunk * kImg + (t & 63u) * 256u;
-    uint32_t *rt = rec + (size_t)(t >> 6) * nchunk * 256u + (t & 63u);
+        // a NaN passes fmaxf by: it goes through the maximum as an infinity
+        if (bad) mx = INFINITY;
 #pragma unroll
-    for (int p = 0; p < PM; p++) {
-        const uint32_t j = tid + 512u * (uint32_t)p;
-        const bool live = j < np;
+        for (int o = 16; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+        bad = !__builtin_isfinite(mx);
+        int E = 0;
+        (void)frexpf(mx, &E);
+        const int e2 = bad || mx == 0.f ? 0 : min(max(10 - E, -126), 126);
+        const float sc = ldexpf(1.0f, e2);
         _Float16 h[8], l[8];
         float s = 0.f;
 #pragma unroll
@@ -648,8 +668,10 @@ __global__ void __launch_bounds__(512) wide_planes_k(const float *__restrict__ a
         *(h8 *)(d + 16384u) = ll;
         if ((j & 3u) == 0u) {
             const _Float16 sh = (_Float16)s, sl = (_Float16)(s - (float)sh);
-            rt[(size_t)(j >> 2) * 64u] = as_u(h2{sh, sl});
+            rt[(j >> 4) * kRec + ((j >> 2) & 3u) * 64u] = as_u(h2{sh, sl});
         }
+        if ((j & 15u) == 0u)
+            rt[(j >> 4) * kRec + 256u] = __builtin_bit_cast(uint32_t, bad ? __builtin_nanf("") : ldexpf(1.0f, -e2));
     }
 }
 
@@ -857,18 +879,17 @@ uint32_t wide_split(uint32_t row_tiles, uint32_t tok_tiles, size_t cols)
 
 template <uint32_t T, bool ONE>
 static void wide_launch(const qgw::Jobs &j, uint32_t tiles, uint32_t tok_tiles, uint32_t slices, uint32_t nchunk,
-                        const uint8_t *xp, const uint32_t *rec, const float *scl, uint32_t ntok, uint32_t ldy,
-                        size_t sstride, hipStream_t st)
+                        const uint8_t *xp, const uint32_t *rec, uint32_t ntok, uint32_t ldy, size_t sstride,
+                        hipStream_t st)
 {
     const uint32_t cps = wide_slice_len(nchunk, slices);
     const dim3 grid((tiles * slices + 7u) / 8u * 8u * tok_tiles);
     hipLaunchKernelGGL((qgw::wide_gemm_k<T, ONE>), grid, dim3(512), qgw::kLds, st, j, tiles, tok_tiles, slices, nchunk,
-                       cps, xp, rec, scl, ntok, ldy, (uint64_t)sstride);
+                       cps, xp, rec, ntok, ldy, (uint64_t)sstride);
 }
 
 int launch_wide_gemm(const PfMat *mats, int n_mats, size_t cols, const uint8_t *xp, const uint32_t *rec,
-                     const float *scl, uint32_t ntok, uint32_t ldy, uint32_t slices, size_t sstride,
-                     ihipStream_t *stream)
+                     uint32_t ntok, uint32_t ldy, uint32_t slices, size_t sstride, ihipStream_t *stream)
 {
     if (ntok == 0) return 0;
     if (n_mats < 1 || n_mats > 3 || ntok > kWideMax || slices < 1 || slices > kWideSlices) return -1;
@@ -887,20 +908,20 @@ int launch_wide_gemm(const PfMat *mats, int n_mats, size_t cols, const uint8_t *
     const bool one = mats[0].g == 1;
     switch (mats[0].type) {
     case T_Q4_K:
-        if (one) wide_launch<T_Q4_K, true>(j, tiles, tt, slices, nchunk, xp, rec, scl, ntok, ldy, sstride, st);
-        else wide_launch<T_Q4_K, false>(j, tiles, tt, slices, nchunk, xp, rec, scl, ntok, ldy, sstride, st);
+        if (one) wide_launch<T_Q4_K, true>(j, tiles, tt, slices, nchunk, xp, rec, ntok, ldy, sstride, st);
+        else wide_launch<T_Q4_K, false>(j, tiles, tt, slices, nchunk, xp, rec, ntok, ldy, sstride, st);
         break;
     case T_Q5_K:
-        if (one) wide_launch<T_Q5_K, true>(j, tiles, tt, slices, nchunk, xp, rec, scl, ntok, ldy, sstride, st);
-        else wide_launch<T_Q5_K, false>(j, tiles, tt, slices, nchunk, xp, rec, scl, ntok, ldy, sstride, st);
+        if (one) wide_launch<T_Q5_K, true>(j, tiles, tt, slices, nchunk, xp, rec, ntok, ldy, sstride, st);
+        else wide_launch<T_Q5_K, false>(j, tiles, tt, slices, nchunk, xp, rec, ntok, ldy, sstride, st);
         break;
     case T_Q6_K:
-        if (one) wide_launch<T_Q6_K, true>(j, tiles, tt, slices, nchunk, xp, rec, scl, ntok, ldy, sstride, st);
-        else wide_launch<T_Q6_K, false>(j, tiles, tt, slices, nchunk, xp, rec, scl, ntok, ldy, sstride, st);
+        if (one) wide_launch<T_Q6_K, true>(j, tiles, tt, slices, nchunk, xp, rec, ntok, ldy, sstride, st);
+        else wide_launch<T_Q6_K, false>(j, tiles, tt, slices, nchunk, xp, rec, ntok, ldy, sstride, st);
         break;
     case T_Q8_0:
         if (!one) return -1;
-        wide_launch<T_Q8_0, true>(j, tiles, tt, slices, nchunk, xp, rec, scl, ntok, ldy, sstride, st);
+        wide_launch<T_Q8_0, true>(j, tiles, tt, slices, nchunk, xp, rec, ntok, ldy, sstride, st);
         break;
     default: return -1;
     }
@@ -909,7 +930,7 @@ int launch_wide_gemm(const PfMat *mats, int n_mats, size_t cols, const uint8_t *
 
 int launch_wide_planes(const float *a, uint32_t na, const float *b, uint32_t nb, size_t sstride, float *sum_out,
                        const float *nw, size_t n, size_t lda, int mode, float eps, uint8_t *xp, uint32_t *rec,
-                       float *scl, uint32_t ntok, ihipStream_t *stream)
+                       uint32_t ntok, ihipStream_t *stream)
 {
     if (ntok == 0) return 0;
     if (n % 128 != 0 || n == 0 || n > kWideCols || ntok > kWideMax || na < 1 || (b && nb < 1) || (mode == 2 && !b) ||
@@ -920,7 +941,7 @@ int launch_wide_planes(const float *a, uint32_t na, const float *b, uint32_t nb,
     const uint32_t pm = (uint32_t)((n / 8 + 511) / 512);
     auto go = [&](auto fn) {
         hipLaunchKernelGGL(fn, dim3(ntok), dim3(512), 0, st, a, na, b, nb, (uint64_t)sstride, sum_out, nw, (uint32_t)n,
-                           (uint32_t)lda, (uint32_t)mode, eps, xp, rec, scl);
+                           (uint32_t)lda, (uint32_t)mode, eps, xp, rec);
     };
     if (pm <= 1) go(qgw::wide_planes_k<1>);
     else if (pm <= 2) go(qgw::wide_planes_k<2>);

@@ -42,6 +42,56 @@ def test_two_chunks_and_continued(rinf, synth, oracle, ctx):
     assert max([e0, e1] + errs + errs1) <= DEEP_TOL, (e0, errs, e1, errs1)
 
 
+class Edited:
+    """synth with gen_model's tensors changed by `edit`."""
+
+    def __init__(self, synth, edit):
+        self.synth, self.edit = synth, edit
+
+    def gen_model(self, cfg, mix, seed):
+        t = self.synth.gen_model(cfg, mix, seed)
+        self.edit(t)
+        return t
+
+
+# byte offsets of the f16 scales (d, and dmin) of a block, elements and bytes of one
+SCALES = {8: ((0,), 32, 34), 12: ((0, 2), 256, 144), 13: ((0, 2), 256, 176), 14: ((208,), 256, 210)}
+
+
+def scale_blocks(mat, first, last, factor):
+    """The scales of the blocks that hold the flat elements first .. last - 1."""
+    raw, dtype, _, _ = mat
+    offsets, be, bb = SCALES[dtype]
+    blocks = raw.reshape(-1, bb)[first // be:-(-last // be)]
+    for o in offsets:
+        f = np.ascontiguousarray(blocks[:, o:o + 2]).view(np.float16)
+        blocks[:, o:o + 2] = (f.astype(np.float32) * factor).astype(np.float16).view(np.uint8)
+
+
+@pytest.mark.parametrize("cfg,mix", [(dict(SMALL, hidden_dim=1024), "q4_k_m"), (dict(SMALL, hidden_dim=1024), "q5_k"),
+                                     (dict(SMALL, hidden_dim=1024), "q8_0"), (HALF, "q4_k_m")])
+def test_outlier(rinf, synth, oracle, ctx, cfg, mix):
+    """One activation 2^40 times the others (row 4 of gate and up 2^20 times the
+    rest) that no output depends on (its 256-element group's weights in down
+    are zero): the other groups keep their 22 bits, as in the 64-token chunks.
+    Under a scale common to the token they would vanish."""
+    def edit(t):
+        for layer in range(cfg["n_layers"]):
+            for slot in ("gate", "up"):
+                scale_blocks(t["mats"][slot, layer], 4 * cfg["embed_dim"], 5 * cfg["embed_dim"], 2.0 ** 20)
+            raw, dtype, rows, cols = t["mats"]["down", layer]
+            for r in range(rows):
+                if dtype == 14:                   # a scale byte per 16 elements
+                    f = np.arange(r * cols, r * cols + 256, 16)
+                    raw.reshape(-1, 210)[f // 256, 192 + f % 256 // 16] = 0
+                else:
+                    scale_blocks(t["mats"]["down", layer], r * cols, r * cols + 256, 0.0)
+
+    for seed in (1, 2, 3):
+        e0, errs, _ = prefill_and_compare(rinf, Edited(synth, edit), oracle, ctx, cfg, mix, seed, 70 + seed, 4, 96)
+        assert e0 <= DEEP_TOL and max(errs) <= DEEP_TOL, (seed, e0, errs)
+
+
 def test_no_room_for_the_wide_buffers(rinf, synth, oracle, ctx):
     """Where the wide chunks' buffers cannot be allocated the prompt goes through
     64-token chunks; the next prompt finds room and takes the wide ones."""
