@@ -92,6 +92,46 @@ def test_outlier(rinf, synth, oracle, ctx, cfg, mix):
         assert e0 <= DEEP_TOL and max(errs) <= DEEP_TOL, (seed, e0, errs)
 
 
+@pytest.mark.parametrize("n", [64, 65])
+def test_q6_k_products_are_exact(rinf, synth, oracle, ctx, n):
+    """Q6_K values of 12 bits (scale -127, code 1: d 3937) against x of two f16
+    pieces, hi + 0.125 each, that sum to zero: v is zero, and only if every
+    product of a piece of x with a piece of the weight is formed (the low
+    pieces' with the weight's last bit sum to 32 d of 64 million).  wo spreads v
+    with alternating signs, so logits other than the all-equal h's show it."""
+    cfg = dict(SMALL, n_layers=1, norm_eps=0.0)
+    E, V = cfg["embed_dim"], cfg["vocab_size"]
+    x = np.where(np.arange(E) % 2 == 0, 1000.125, -999.875)
+    x[0:32:2] -= 2.0
+    assert x.sum() == 0
+
+    def edit(t):
+        for slot in ("wq", "wk", "wv", "gate", "up", "down"):
+            scale_blocks(t["mats"][slot, 0], 0, int(np.prod(t["mats"][slot, 0][2:])), 0.0)
+        emb = t["mats"]["token_embd", 0]
+        t["mats"]["token_embd", 0] = (np.ones(V * E, np.float32).view(np.uint8), 0, V, E)
+        wv = t["mats"]["wv", 0][0].reshape(-1, 210)
+        wv[:, :128], wv[:, 128:192], wv[:, 192:208] = 0x11, 0, 0x81
+        wv[:, 208:210] = np.array([256.0], np.float16).view(np.uint8)
+        wo = t["mats"]["wo", 0][0].reshape(E, 144)                  # one block a row: d = +-2^-6, codes 1, mins 0
+        wo[:, 0:2] = np.where(np.arange(E) % 2 == 0, 2.0 ** -6, -2.0 ** -6).astype(np.float16).view(np.uint8).reshape(E, 2)
+        wo[:, 2:4], wo[:, 4:8], wo[:, 8:12], wo[:, 12:16], wo[:, 16:] = 0, 1, 0, 1, 0x11
+        assert emb[2:] == (V, E)
+        t["vecs"]["attn_norm", 0] = x.astype(np.float32)
+        for b in ("bq", "bk", "bv"):
+            t["vecs"][b, 0][:] = 0
+
+    dev, _, _ = build(rinf, Edited(synth, edit), oracle, ctx, cfg, "q4_k_m", 21, 96)
+    logits = np.zeros(V, np.float32)
+    dev.prefill(np.arange(n), logits)
+    dev.close()
+    t = synth.gen_model(cfg, "q4_k_m", 21)
+    raw, dtype, rows, cols = t["mats"]["lm_head", 0]
+    ref = oracle.mat_vec_mul(raw, dtype, rows, cols, t["vecs"]["final_norm", 0])
+    err = normwise_err(logits, ref)
+    assert err <= DEEP_TOL, err
+
+
 def test_no_room_for_the_wide_buffers(rinf, synth, oracle, ctx):
     """Where the wide chunks' buffers cannot be allocated the prompt goes through
     64-token chunks; the next prompt finds room and takes the wide ones."""
