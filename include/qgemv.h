@@ -207,7 +207,7 @@ int qg_set_precision(qg_ctx *ctx, int mode);
 
 /* Test hook, no counterpart in the reference: of the allocations this
  * context makes next (device matrices, repacked and stacked copies, pinned
- * and device staging), the first `skip` go through and the `n` after them
+ * and device staging, a model's buffers), the first `skip` go through and the `n` after them
  * report QG_ERR_OUT_OF_MEMORY without calling HIP, so that tests can drive
  * the status-code path a caller maps to its CPU fallback
  * (gpu_backend.rs:444-447) without a device fault.  n = 0 switches it off. */

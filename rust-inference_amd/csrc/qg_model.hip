@@ -829,6 +829,7 @@ struct qg_model {
     // planes / records of the GEMMs and the prompt's token ids; allocated on
     // first use
     bool pf_batched = true;
+    bool pf_ready = false;                // all of them allocated
     float *pf_h[2] = {nullptr, nullptr}, *pf_qkv = nullptr, *pf_ao = nullptr, *pf_ao2 = nullptr,
           *pf_g = nullptr, *pf_fo = nullptr, *pf_last = nullptr;
     uint16_t *pf_xp = nullptr;
@@ -878,14 +879,26 @@ int mfail(qg_model *m, int st, const char *what, hipError_t e = hipSuccess)
 template <class T> int dalloc(qg_model *m, T **p, size_t n)
 {
     void *d = nullptr;
-    hipError_t e = hipMalloc(&d, (n ? n : 1) * sizeof(T));
-    if (e != hipSuccess) return mfail(m, QG_ERR_OUT_OF_MEMORY, "hipMalloc", e);
+    hipError_t e = qg_alloc_injected(m->ctx) ? hipErrorOutOfMemory : hipMalloc(&d, (n ? n : 1) * sizeof(T));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return mfail(m, QG_ERR_OUT_OF_MEMORY, "hipMalloc", e);
+    }
     e = hipMemsetAsync(d, 0, (n ? n : 1) * sizeof(T), m->ctx->stream);
     if (e != hipSuccess) { (void)hipFree(d); return mfail(m, QG_ERR_HIP, "hipMemsetAsync", e); }
     m->allocs.push_back(d);
     m->alloc_bytes += (n ? n : 1) * sizeof(T);
     *p = (T *)d;
     return QG_OK;
+}
+
+// Gives back what dalloc handed out after the first `held` allocations (of
+// `bytes` bytes): a set of buffers is there as a whole or not at all.
+void undo_allocs(qg_model *m, size_t held, size_t bytes)
+{
+    (void)hipStreamSynchronize(m->ctx->stream);
+    for (; m->allocs.size() > held; m->allocs.pop_back()) (void)hipFree(m->allocs.back());
+    m->alloc_bytes = bytes;
 }
 
 // hipMemcpy in the order of the context's stream, and waited for.  The legacy
@@ -1376,7 +1389,7 @@ bool pf_supported(const qg_model *m)
 
 int pf_alloc(qg_model *m)
 {
-    if (m->pf_h[0]) return QG_OK;
+    if (m->pf_ready) return QG_OK;
     const size_t T = qg::kPfMaxTokens, E = m->cfg.embed_dim, H = m->cfg.hidden_dim;
     const size_t ldq = m->q_dim + 2 * (size_t)m->kv_dim;
     size_t kmax = E > H ? E : H;
@@ -1390,6 +1403,7 @@ int pf_alloc(qg_model *m)
     m->pf_s_o = qg::pf_split(qg::pf_tiles(E), (uint32_t)(m->q_dim / 32));
     m->pf_s_gu = qg::pf_split(2 * qg::pf_tiles(H), (uint32_t)(E / 32));
     m->pf_s_down = qg::pf_split(qg::pf_tiles(E), (uint32_t)(H / 32));
+    const size_t held = m->allocs.size(), bytes = m->alloc_bytes;
     int rc;
     if ((rc = dalloc(m, &m->pf_h[0], T * E)) || (rc = dalloc(m, &m->pf_h[1], T * E)) ||
         (rc = dalloc(m, &m->pf_qkv, m->pf_s_qkv * T * ldq)) || (rc = dalloc(m, &m->pf_ao, T * m->q_dim)) ||
@@ -1398,8 +1412,11 @@ int pf_alloc(qg_model *m)
         (rc = dalloc(m, &m->pf_xp, 2 * T * kmax)) ||
         (rc = dalloc(m, &m->pf_rec, T * (kmax / 32 + (kmax + 255) / 256))) ||
         (rc = dalloc(m, &m->pf_ss, T * ((E + 255) / 256))) ||
-        (rc = dalloc(m, &m->pf_tok, (size_t)m->cfg.max_seq_len)))
+        (rc = dalloc(m, &m->pf_tok, (size_t)m->cfg.max_seq_len))) {
+        undo_allocs(m, held, bytes);
         return rc;
+    }
+    m->pf_ready = true;
     return QG_OK;
 }
 
@@ -1561,18 +1578,12 @@ int wide_alloc(qg_model *m)
     }
     const size_t held = m->allocs.size(), bytes = m->alloc_bytes;
     int rc;
-    if (qg_alloc_injected(m->ctx)) rc = mfail(m, QG_ERR_OUT_OF_MEMORY, "hipMalloc (injected failure)");
-    else if ((rc = dalloc(m, &m->wd_h[0], T * E)) || (rc = dalloc(m, &m->wd_h[1], T * E)) ||
-             (rc = dalloc(m, &m->wd_qkv, rq * ldq)) || (rc = dalloc(m, &m->wd_ao, T * m->q_dim)) ||
-             (rc = dalloc(m, &m->wd_ao2, ro * E)) || (rc = dalloc(m, &m->wd_g, rg * 2 * H)) ||
-             (rc = dalloc(m, &m->wd_fo, rd * E)) || (rc = dalloc(m, &m->wd_xp, T * kmax * 4)))
-        ;
-    else rc = dalloc(m, &m->wd_rec, T * kmax / 128 * 5);
-    if (rc) {                                            // all of them or none
-        (void)hipGetLastError();
-        (void)hipStreamSynchronize(m->ctx->stream);
-        for (; m->allocs.size() > held; m->allocs.pop_back()) (void)hipFree(m->allocs.back());
-        m->alloc_bytes = bytes;
+    if ((rc = dalloc(m, &m->wd_h[0], T * E)) || (rc = dalloc(m, &m->wd_h[1], T * E)) ||
+        (rc = dalloc(m, &m->wd_qkv, rq * ldq)) || (rc = dalloc(m, &m->wd_ao, T * m->q_dim)) ||
+        (rc = dalloc(m, &m->wd_ao2, ro * E)) || (rc = dalloc(m, &m->wd_g, rg * 2 * H)) ||
+        (rc = dalloc(m, &m->wd_fo, rd * E)) || (rc = dalloc(m, &m->wd_xp, T * kmax * 4)) ||
+        (rc = dalloc(m, &m->wd_rec, T * kmax / 128 * 5))) {
+        undo_allocs(m, held, bytes);
         return rc;
     }
     m->pf_wide = cap;

@@ -151,3 +151,44 @@ def test_no_room_for_the_wide_buffers(rinf, synth, oracle, ctx):
     dev.close()
     if shared is not None:
         shared.free()
+
+
+def test_every_failed_allocation(rinf, synth, oracle, ctx):
+    """Each allocation of a prefill fails in turn.  Of the buffers every prefill
+    needs: out of memory, nothing kept, and the next call starts over.  Of the
+    wide chunks': the prompt goes through 64-token chunks, and the buffers
+    before the failed one are given back."""
+    cfg = dict(SMALL, n_layers=1)
+    dev, ref, _ = build(rinf, synth, oracle, ctx, cfg, "q4_k_m", 12, 96)
+    prompt = np.random.default_rng(12).integers(0, cfg["vocab_size"], 70)
+    for pos, tok in enumerate(prompt):
+        ref_l = ref.forward(int(tok), pos)
+    logits = np.zeros(cfg["vocab_size"], np.float32)
+
+    def attempt(skip):
+        dev.reset()
+        logits[:] = 0
+        ctx.fail_allocations(1, skip)
+        try:
+            dev.prefill(prompt, logits)
+        finally:
+            ctx.fail_allocations(0)
+        assert normwise_err(logits, ref_l) <= DEEP_TOL, skip
+
+    failed = 0
+    for skip in range(64):
+        try:
+            attempt(skip)
+            break
+        except rinf.QgemvError as e:
+            assert e.status == 6, e
+            failed += 1
+            assert dev.seq_len == 0
+    assert failed >= 12                           # qg_model.hip, pf_alloc
+    held = dev.resident_bytes()
+    for skip in range(64):                        # wide_alloc, until all of them go through
+        attempt(skip)
+        if dev.resident_bytes() != held:
+            break
+    assert 1 <= skip < 63
+    dev.close()
