@@ -1684,9 +1684,11 @@ int prefill(qg_model *m, const uint32_t *tok, size_t n)
         // whole tiles), where every matrix takes them and the card has room
         // for their buffers
         bool wide = n > qg::kPfMaxTokens && wide_supported(m);
+        const std::string err = m->ctx->err;
         if (wide && (rc = wide_alloc(m))) {
             if (rc != QG_ERR_OUT_OF_MEMORY) return rc;
             wide = false;
+            m->ctx->err = err;                           // this call has not failed
         }
         size_t len = qg::kPfMaxTokens;
         if (wide) {

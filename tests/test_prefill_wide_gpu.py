@@ -134,16 +134,21 @@ def test_q6_k_products_are_exact(rinf, synth, oracle, ctx, n):
 
 def test_no_room_for_the_wide_buffers(rinf, synth, oracle, ctx):
     """Where the wide chunks' buffers cannot be allocated the prompt goes through
-    64-token chunks; the next prompt finds room and takes the wide ones."""
+    64-token chunks; the next prompt finds room and takes the wide ones.  The
+    context's last error stays the one of the call before them."""
     dev, ref, shared = build(rinf, synth, oracle, ctx, SMALL, "q4_k_m", 11, 400)
     prompt = np.random.default_rng(11).integers(0, SMALL["vocab_size"], 330)
     logits = np.zeros(SMALL["vocab_size"], np.float32)
     pos = 0
+    with pytest.raises(rinf.QgemvError):
+        dev.prefill([SMALL["vocab_size"]])
+    last_error = ctx.lib.qg_last_error(ctx.h)
     for part, fail in ((prompt[:40], False), (prompt[40:190], True), (prompt[190:], False)):
         if fail:
             ctx.fail_allocations(1)
         dev.prefill(part, logits)
         ctx.fail_allocations(0)
+        assert ctx.lib.qg_last_error(ctx.h) == last_error
         for tok in part:
             ref_l = ref.forward(int(tok), pos)
             pos += 1
