@@ -30,6 +30,7 @@
 //   sample_final_k   of the logits per workgroup; then the first maximum
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -839,11 +840,17 @@ struct qg_model {
     // the QKV output's K splits: [Q; K; V] in one launch (one type), or
     // [Q; K] and V in two (V another type: its few row tiles take more slices)
     uint32_t pf_s_qkv1 = 1, pf_s_qk = 1, pf_s_v = 1;
-    // prefill of more than kPfMaxTokens tokens (qg_prefill_wide.hip), up to
-    // pf_wide tokens per chunk: the same buffers for whole tiles of tokens
-    uint32_t pf_wide = 0;
-    float *wd_h[2] = {nullptr, nullptr}, *wd_qkv = nullptr, *wd_ao = nullptr, *wd_ao2 = nullptr, *wd_g = nullptr,
-          *wd_fo = nullptr;
+    // prefill of more than kPfMaxTokens tokens (qg_prefill_wide.hip): the same
+    // buffers in one allocation wd_mem, for chunks of up to wd_cap tokens (whole
+    // tiles), as long as the prompts so far needed; wd_v: V's GEMM output in
+    // the layers that have it apart from Q's and K's, wd_qkv (rows of wd_ldq
+    // floats): with V where a layer has the three in one launch
+    bool wd_apart = false, wd_joined = false;
+    uint32_t wd_cap = 0, wd_ldq = 0;
+    size_t wd_bytes = 0;
+    float *wd_mem = nullptr;
+    float *wd_h[2] = {nullptr, nullptr}, *wd_qkv = nullptr, *wd_v = nullptr, *wd_ao = nullptr, *wd_ao2 = nullptr,
+          *wd_g = nullptr, *wd_fo = nullptr;
     uint8_t *wd_xp = nullptr;
     uint32_t *wd_rec = nullptr;
     // captured graphs per attention mode: [0] the split attention
@@ -1508,7 +1515,8 @@ int pf_chunk(qg_model *m, const uint32_t *d_tok, uint32_t ntok, uint32_t s0, boo
             return rc;
         }
         float *kc = m->kc + l * kv_layer, *vc = m->vc + l * kv_layer;
-        if (qg::launch_pf_qkv_post(m->pf_qkv, ldq, s_qk, s_v, T * ldq, m->pf_ss, E, c.norm_eps,
+        if (qg::launch_pf_qkv_post(m->pf_qkv, ldq, s_qk, T * ldq, m->pf_qkv + m->q_dim + m->kv_dim, ldq, s_v, T * ldq,
+                                   m->pf_ss, E, c.norm_eps,
                                    m->vec[QG_V_BQ][l], m->vec[QG_V_BK][l], m->vec[QG_V_BV][l], kc, vc, m->cos_t,
                                    m->sin_t, m->q_dim, m->kv_dim, m->hd, s0, s0, ntok, sti) ||
             qg::launch_pf_attention(m->pf_qkv, ldq, kc, vc, m->pf_ao, c.n_heads, m->hd, m->kv_dim, m->n_rep, scale, s0,
@@ -1560,33 +1568,62 @@ WideSplit wide_splits(const qg_model *m, uint32_t tt)
                      qg::wide_split(te, tt, H)};
 }
 
-int wide_alloc(qg_model *m)
+// V takes a launch of its own: another type or row grouping than K
+bool wide_v_apart(const qg_model *m, uint32_t l)
 {
-    if (m->pf_wide) return QG_OK;
-    const size_t E = m->cfg.embed_dim, H = m->cfg.hidden_dim, ldq = m->q_dim + 2 * (size_t)m->kv_dim;
-    const uint32_t cap = std::min<uint32_t>(qg::kWideMax, (m->cfg.max_seq_len + qg::kWideTile - 1) / qg::kWideTile * qg::kWideTile);
-    const size_t kmax = std::max({E, H, (size_t)m->q_dim}), T = cap;
+    const qg_mat *k = m->w[QG_M_WK - 2][l], *v = m->w[QG_M_WV - 2][l];
+    return k->type != v->type || (k->plan.g == 1) != (v->plan.g == 1);
+}
+
+// The buffers for wide chunks of `tokens` tokens, and for the layers' matrices
+// as they are now (a slot may have got one of another type since the last
+// prompt).  They grow with the longest chunk so far (Qwen2-7B: 79 MB for a prompt of 65 tokens, 425 MB for 1024).
+int wide_alloc(qg_model *m, size_t tokens)
+{
+    const uint32_t cap = (uint32_t)((tokens + qg::kWideTile - 1) / qg::kWideTile * qg::kWideTile);
+    bool apart = false, joined = false;
+    for (uint32_t l = 0; l < m->cfg.n_layers; l++) (wide_v_apart(m, l) ? apart : joined) = true;
+    if (cap <= m->wd_cap && (m->wd_apart || !apart) && (m->wd_joined || !joined)) return QG_OK;
+    if (m->wd_mem) {
+        (void)hipStreamSynchronize(m->ctx->stream);
+        m->allocs.erase(std::find(m->allocs.begin(), m->allocs.end(), (void *)m->wd_mem));
+        m->alloc_bytes -= m->wd_bytes;
+        (void)hipFree(m->wd_mem);
+        m->wd_mem = nullptr;
+        m->wd_cap = 0;
+    }
+    const size_t E = m->cfg.embed_dim, H = m->cfg.hidden_dim, kmax = std::max({E, H, (size_t)m->q_dim}), T = cap;
+    m->wd_ldq = m->q_dim + m->kv_dim + (joined ? m->kv_dim : 0);
     // rows of the GEMM outputs: their slices at every number of token tiles
-    size_t rq = 0, ro = 0, rg = 0, rd = 0;
+    size_t rq = 0, rv = 0, ro = 0, rg = 0, rd = 0;
     for (uint32_t tt = 1; tt <= cap / qg::kWideTile; tt++) {
         const WideSplit s = wide_splits(m, tt);
         const size_t t = (size_t)tt * qg::kWideTile;
-        rq = std::max(rq, t * std::max({s.qkv, s.qk, s.v}));
+        rq = std::max(rq, t * std::max(joined ? s.qkv : 0u, apart ? s.qk : 0u));
+        rv = std::max(rv, apart ? t * s.v : 0);
         ro = std::max(ro, t * s.o);
         rg = std::max(rg, t * s.gu);
         rd = std::max(rd, t * s.down);
     }
-    const size_t held = m->allocs.size(), bytes = m->alloc_bytes;
-    int rc;
-    if ((rc = dalloc(m, &m->wd_h[0], T * E)) || (rc = dalloc(m, &m->wd_h[1], T * E)) ||
-        (rc = dalloc(m, &m->wd_qkv, rq * ldq)) || (rc = dalloc(m, &m->wd_ao, T * m->q_dim)) ||
-        (rc = dalloc(m, &m->wd_ao2, ro * E)) || (rc = dalloc(m, &m->wd_g, rg * 2 * H)) ||
-        (rc = dalloc(m, &m->wd_fo, rd * E)) || (rc = dalloc(m, &m->wd_xp, T * kmax * 4)) ||
-        (rc = dalloc(m, &m->wd_rec, T * kmax / 128 * 5))) {
-        undo_allocs(m, held, bytes);
-        return rc;
-    }
-    m->pf_wide = cap;
+    // (every part a multiple of 128 floats: the rows are whole tiles of tokens)
+    const size_t sizes[10] = {T * E, T * E, rq * m->wd_ldq, rv * m->kv_dim, T * m->q_dim, ro * E, rg * 2 * H, rd * E,
+                              T * kmax, T * kmax / 128 * 5};
+    size_t total = 0;
+    for (size_t n : sizes) total += n;
+    const size_t bytes = m->alloc_bytes;
+    if (int rc = dalloc(m, &m->wd_mem, total)) return rc;
+    m->wd_bytes = m->alloc_bytes - bytes;
+    float *p = m->wd_mem;
+    auto take = [&](int i) { float *q = p; p += sizes[i]; return q; };
+    m->wd_h[0] = take(0); m->wd_h[1] = take(1);
+    m->wd_qkv = take(2); m->wd_v = take(3);
+    m->wd_ao = take(4); m->wd_ao2 = take(5);
+    m->wd_g = take(6); m->wd_fo = take(7);
+    m->wd_xp = (uint8_t *)take(8);
+    m->wd_rec = (uint32_t *)take(9);
+    m->wd_cap = cap;
+    m->wd_apart = apart;
+    m->wd_joined = joined;
     return QG_OK;
 }
 
@@ -1614,12 +1651,12 @@ int wide_planes(qg_model *m, const float *a, uint32_t na, const float *b, uint32
     return QG_OK;
 }
 
-// pf_chunk for up to m->pf_wide tokens
+// pf_chunk for up to m->wd_cap tokens
 int wide_chunk(qg_model *m, const uint32_t *d_tok, uint32_t ntok, uint32_t s0, bool last)
 {
     const qg_model_config &c = m->cfg;
     ihipStream_t *sti = (ihipStream_t *)m->ctx->stream;
-    const uint32_t E = c.embed_dim, H = c.hidden_dim, ldq = m->q_dim + 2 * m->kv_dim;
+    const uint32_t E = c.embed_dim, H = c.hidden_dim, ldq = m->wd_ldq;
     const uint32_t tt = (ntok + qg::kWideTile - 1) / qg::kWideTile;
     const WideSplit sp = wide_splits(m, tt);
     const size_t T = (size_t)tt * qg::kWideTile;
@@ -1637,17 +1674,19 @@ int wide_chunk(qg_model *m, const uint32_t *d_tok, uint32_t ntok, uint32_t s0, b
                               m->vec[QG_V_ATTN_NORM][l], E, E, 1, ntok)))
             return rc;
         if (l) std::swap(h, h2);
+        const bool v_apart = wide_v_apart(m, l);
+        const uint32_t s_qk = v_apart ? sp.qk : sp.qkv, s_v = v_apart ? sp.v : sp.qkv;
+        float *v = v_apart ? m->wd_v : m->wd_qkv + m->q_dim + m->kv_dim;
+        const uint32_t ldv = v_apart ? m->kv_dim : ldq;
         const qg::PfMat qkv[3] = {pf_mat(m->w[QG_M_WQ - 2][l], m->wd_qkv),
                                   pf_mat(m->w[QG_M_WK - 2][l], m->wd_qkv + m->q_dim),
-                                  pf_mat(m->w[QG_M_WV - 2][l], m->wd_qkv + m->q_dim + m->kv_dim)};
-        const bool v_apart = qkv[2].type != qkv[1].type || (qkv[2].g == 1) != (qkv[1].g == 1);
-        const uint32_t s_qk = v_apart ? sp.qk : sp.qkv, s_v = v_apart ? sp.v : sp.qkv;
+                                  pf_mat(m->w[QG_M_WV - 2][l], v)};
         if ((rc = wide_gemm(m, qkv, v_apart ? 2 : 3, E, ntok, ldq, s_qk, T * ldq)) ||
-            (v_apart && (rc = wide_gemm(m, qkv + 2, 1, E, ntok, ldq, s_v, T * ldq))))
+            (v_apart && (rc = wide_gemm(m, qkv + 2, 1, E, ntok, ldv, s_v, T * ldv))))
             return rc;
         float *kc = m->kc + l * kv_layer, *vc = m->vc + l * kv_layer;
-        if (qg::launch_pf_qkv_post(m->wd_qkv, ldq, s_qk, s_v, T * ldq, nullptr, E, c.norm_eps, m->vec[QG_V_BQ][l],
-                                   m->vec[QG_V_BK][l], m->vec[QG_V_BV][l], kc, vc, m->cos_t, m->sin_t, m->q_dim,
+        if (qg::launch_pf_qkv_post(m->wd_qkv, ldq, s_qk, T * ldq, v, ldv, s_v, T * ldv, nullptr, E, c.norm_eps,
+                                   m->vec[QG_V_BQ][l], m->vec[QG_V_BK][l], m->vec[QG_V_BV][l], kc, vc, m->cos_t, m->sin_t, m->q_dim,
                                    m->kv_dim, m->hd, s0, s0, ntok, sti) ||
             qg::launch_wide_attention(m->wd_qkv, ldq, kc, vc, m->wd_ao, c.n_heads, m->hd, m->kv_dim, m->n_rep, scale,
                                       s0, ntok, sti))
@@ -1684,16 +1723,17 @@ int prefill(qg_model *m, const uint32_t *tok, size_t n)
         // whole tiles), where every matrix takes them and the card has room
         // for their buffers
         bool wide = n > qg::kPfMaxTokens && wide_supported(m);
-        const std::string err = m->ctx->err;
-        if (wide && (rc = wide_alloc(m))) {
-            if (rc != QG_ERR_OUT_OF_MEMORY) return rc;
-            wide = false;
-            m->ctx->err = err;                           // this call has not failed
-        }
         size_t len = qg::kPfMaxTokens;
         if (wide) {
-            const size_t parts = (n + m->pf_wide - 1) / m->pf_wide, per = (n + parts - 1) / parts;
-            len = (per + qg::kWideTile - 1) / qg::kWideTile * qg::kWideTile;
+            const size_t parts = (n + qg::kWideMax - 1) / qg::kWideMax, per = (n + parts - 1) / parts;
+            const std::string err = m->ctx->err;
+            if ((rc = wide_alloc(m, per)) == QG_OK) {
+                len = (per + qg::kWideTile - 1) / qg::kWideTile * qg::kWideTile;
+            } else {
+                if (rc != QG_ERR_OUT_OF_MEMORY) return rc;
+                wide = false;
+                m->ctx->err = err;                       // this call has not failed
+            }
         }
         for (size_t i = 0; i < n; i += len) {
             const uint32_t nt = (uint32_t)std::min(n - i, len);

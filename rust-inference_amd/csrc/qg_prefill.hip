@@ -1199,12 +1199,13 @@ __global__ void __launch_bounds__(256) pf_sum_k(const float *__restrict__ x, uin
 // ----------------------------------------------------- attention, post-ops
 
 // Bias add, RoPE and KV append of token t of the chunk (position pos0 + t,
-// cache slot slot0 + t); q, k, v of a token are contiguous with stride ldq,
-// summed over the ns K-split slices of the QKV GEMM (sstride floats apart);
-// the rotated q goes to slice 0.  The expressions of the decode path's
-// qkv_post_k.
-__global__ void __launch_bounds__(256) pf_qkv_post_k(float *__restrict__ qkv, uint32_t ldq, uint32_t ns,
-                                                     uint32_t ns_v, uint64_t sstride, const float *__restrict__ ss,
+// cache slot slot0 + t); q and k of a token are contiguous with stride ldq,
+// summed over the ns K-split slices of their GEMM (sstride floats apart), v
+// has its own place, stride and slices; the rotated q goes to slice 0.  The
+// expressions of the decode path's qkv_post_k.
+__global__ void __launch_bounds__(256) pf_qkv_post_k(float *__restrict__ qk, uint32_t ldq, uint32_t ns,
+                                                     uint64_t sstride, const float *__restrict__ va, uint32_t ldv,
+                                                     uint32_t ns_v, uint64_t vstride, const float *__restrict__ ss,
                                                      uint32_t ss_ng,
                                                      uint32_t ss_n, float eps, const float *__restrict__ bq,
                                                      const float *__restrict__ bk, const float *__restrict__ bv,
@@ -1215,7 +1216,8 @@ __global__ void __launch_bounds__(256) pf_qkv_post_k(float *__restrict__ qkv, ui
 {
     const uint32_t t = blockIdx.y, i0 = 2 * (blockIdx.x * blockDim.x + threadIdx.x), half = hd / 2;
     const uint32_t pos = pos0 + t, slot = slot0 + t;
-    float *q = qkv + (size_t)t * ldq, *k = q + q_dim, *v = k + kv_dim;
+    float *q = qk + (size_t)t * ldq, *k = q + q_dim;
+    const float *v = va + (size_t)t * ldv;
     // the GEMM took the norm's numerator: its 1 / rms here, before the biases
     const float r = ss ? pf_inv_rms(ss, ss_ng, t, ss_n, eps) : 1.0f;
     if (i0 < q_dim) {
@@ -1234,8 +1236,8 @@ __global__ void __launch_bounds__(256) pf_qkv_post_k(float *__restrict__ qkv, ui
         float *kr = kc + (size_t)slot * kv_dim, *vr = vc + (size_t)slot * kv_dim;
         kr[i0] = x0 * c - x1 * s;
         kr[i0 + 1] = x0 * s + x1 * c;
-        vr[i0] = sum_slices(v + i0, ns_v, sstride) * r + bv[i0];
-        vr[i0 + 1] = sum_slices(v + i0 + 1, ns_v, sstride) * r + bv[i0 + 1];
+        vr[i0] = sum_slices(v + i0, ns_v, vstride) * r + bv[i0];
+        vr[i0 + 1] = sum_slices(v + i0 + 1, ns_v, vstride) * r + bv[i0 + 1];
     }
 }
 
@@ -1519,8 +1521,8 @@ int launch_pf_sum(const float *x, uint32_t ns, size_t sstride, size_t n, float *
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_pf_qkv_post(float *qkv, uint32_t ldq, uint32_t ns, uint32_t ns_v, size_t sstride, const float *ss,
-                       size_t ss_n, float eps,
+int launch_pf_qkv_post(float *qk, uint32_t ldq, uint32_t ns, size_t sstride, const float *v, uint32_t ldv,
+                       uint32_t ns_v, size_t vstride, const float *ss, size_t ss_n, float eps,
                        const float *bq, const float *bk, const float *bv, float *kc, float *vc, const float *cos_t,
                        const float *sin_t, uint32_t q_dim, uint32_t kv_dim, uint32_t hd, uint32_t pos0, uint32_t slot0,
                        uint32_t ntok, ihipStream_t *stream)
@@ -1530,8 +1532,8 @@ int launch_pf_qkv_post(float *qkv, uint32_t ldq, uint32_t ns, uint32_t ns_v, siz
         hd % 2 != 0 || (ss && ss_n == 0) || ss_n > 0xFFFFFFFFull)
         return -1;
     const uint32_t pairs = (q_dim > kv_dim ? q_dim : kv_dim) / 2;
-    hipLaunchKernelGGL(qgp::pf_qkv_post_k, dim3((pairs + 255) / 256, ntok), dim3(256), 0, (hipStream_t)stream, qkv,
-                       ldq, ns, ns_v, (uint64_t)sstride, ss, (uint32_t)((ss_n + 255) / 256), (uint32_t)ss_n, eps, bq, bk, bv,
+    hipLaunchKernelGGL(qgp::pf_qkv_post_k, dim3((pairs + 255) / 256, ntok), dim3(256), 0, (hipStream_t)stream, qk,
+                       ldq, ns, (uint64_t)sstride, v, ldv, ns_v, (uint64_t)vstride, ss, (uint32_t)((ss_n + 255) / 256), (uint32_t)ss_n, eps, bq, bk, bv,
                        kc, vc, cos_t, sin_t, q_dim, kv_dim, hd, pos0, slot0);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }

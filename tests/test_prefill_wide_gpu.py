@@ -197,3 +197,35 @@ def test_every_failed_allocation(rinf, synth, oracle, ctx):
             break
     assert 1 <= skip < 63
     dev.close()
+
+
+def test_buffers_follow_the_prompts(rinf, synth, oracle, ctx):
+    """The wide chunks' buffers are as long as the prompts so far need and not as
+    long as the cache, and fit the layers' matrices as they are: V apart from Q
+    and K (Q6_K, Q4_K), then, with another matrix in its slot, beside them in one
+    launch of the first layer."""
+    dev, ref, _ = build(rinf, synth, oracle, ctx, SMALL, "q4_k_m", 14, 1024)
+    logits = np.zeros(SMALL["vocab_size"], np.float32)
+    rng = np.random.default_rng(14)
+
+    def run(n):
+        prompt = rng.integers(0, SMALL["vocab_size"], n)
+        dev.reset()
+        ref.reset()
+        dev.prefill(prompt, logits)
+        for pos, tok in enumerate(prompt):
+            ref_l = ref.forward(int(tok), pos)
+        assert normwise_err(logits, ref_l) <= DEEP_TOL, n
+        return dev.resident_bytes()["total"]
+
+    bytes_ = [run(n) for n in (20, 65, 300, 128, 900, 70)]
+    narrow, short, middle, _, most, _ = bytes_
+    assert narrow < short < middle < most and bytes_[3] == middle and bytes_[5] == most
+    assert 4 * (short - narrow) < most - narrow
+    kv, E = SMALL["n_kv_heads"] * 64, SMALL["embed_dim"]
+    raw = synth.gen_weights(12, kv, E, 5)
+    dev.set_matrix(rinf.M_WV, 0, raw, 12, kv, E)
+    ref.set_mat("wv", 0, raw, 12, kv, E)
+    for n in (130, 65, 400):
+        run(n)
+    dev.close()
