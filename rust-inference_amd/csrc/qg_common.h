@@ -214,7 +214,8 @@ constexpr uint32_t kWideMax = 1024, kWideCols = 32768, kWideSlices = 8, kWideTil
 bool wide_mat_ok(const PfMat &m, size_t cols);
 uint32_t wide_tiles(size_t rows);
 // slices for row_tiles x tok_tiles workgroup tiles of a GEMM over cols columns
-uint32_t wide_split(uint32_t row_tiles, uint32_t tok_tiles, size_t cols);
+// on n_cu compute units
+uint32_t wide_split(uint32_t row_tiles, uint32_t tok_tiles, size_t cols, int n_cu);
 // 1..3 matrices of one type (and all or none with one row per group) over the
 // same x; slice s of a result at y + s * sstride, y[t * ldy + r]
 int launch_wide_gemm(const PfMat *mats, int n_mats, size_t cols, const uint8_t *xp, const uint32_t *rec,

@@ -1563,9 +1563,9 @@ WideSplit wide_splits(const qg_model *m, uint32_t tt)
 {
     const size_t E = m->cfg.embed_dim, H = m->cfg.hidden_dim;
     const uint32_t tq = qg::wide_tiles(m->q_dim), tk = qg::wide_tiles(m->kv_dim), te = qg::wide_tiles(E);
-    return WideSplit{qg::wide_split(tq + 2 * tk, tt, E), qg::wide_split(tq + tk, tt, E), qg::wide_split(tk, tt, E),
-                     qg::wide_split(te, tt, m->q_dim), qg::wide_split(2 * qg::wide_tiles(H), tt, E),
-                     qg::wide_split(te, tt, H)};
+    auto split = [&](uint32_t rows, size_t cols) { return qg::wide_split(rows, tt, cols, m->ctx->n_cu); };
+    return WideSplit{split(tq + 2 * tk, E), split(tq + tk, E), split(tk, E), split(te, m->q_dim),
+                     split(2 * qg::wide_tiles(H), E), split(te, H)};
 }
 
 // V takes a launch of its own: another type or row grouping than K

@@ -861,18 +861,18 @@ static uint32_t wide_slice_len(uint32_t nchunk, uint32_t slices)
     return nchunk % 2u ? (nchunk + slices - 1u) / slices : 2u * b;
 }
 
-// One workgroup per CU at a time: rounds of 256 workgroups, each as long as
+// One workgroup per CU at a time: rounds of n_cu workgroups, each as long as
 // its slice's blocks plus what a slice costs beside them (filling the
 // pipeline, writing 128 KB of products and reading them back: about 4
 // blocks' time).
-uint32_t wide_split(uint32_t row_tiles, uint32_t tok_tiles, size_t cols)
+uint32_t wide_split(uint32_t row_tiles, uint32_t tok_tiles, size_t cols, int n_cu)
 {
-    const uint32_t nchunk = (uint32_t)(cols / 128u), tiles = row_tiles * tok_tiles;
+    const uint32_t nchunk = (uint32_t)(cols / 128u), tiles = row_tiles * tok_tiles, ncu = n_cu > 0 ? (uint32_t)n_cu : 256u;
     uint32_t best = 1, cost = 0xFFFFFFFFu;
     for (uint32_t s = 1; s <= kWideSlices; s++) {
         const uint32_t len = wide_slice_len(nchunk, s);
         if (len == 0 || (nchunk + len - 1u) / len != s) continue;         // no empty slice
-        const uint32_t c = ((tiles * s + 255u) / 256u) * (len + 8u);
+        const uint32_t c = ((tiles * s + ncu - 1u) / ncu) * (len + 8u);
         if (c < cost) {
             cost = c;
             best = s;
