@@ -620,8 +620,8 @@ class DeviceModel:
 
     def set_attention_path(self, path: int):
         """0: by length (up to 512 cached positions two workgroups per head
-        merged in the wo GEMV where every wo allows it, else up to 256 one;
-        beyond, split), 1: always one workgroup per head, 2: always split over
+        merged in the wo GEMV where every wo allows it, else one up to 288,
+        320 or 480 of them (head_dim 64, 128, 256); beyond, split), 1: always one workgroup per head, 2: always split over
         position ranges, 3: always two workgroups per head where allowed."""
         self.ctx.check(self.ctx.lib.qg_model_set_attention_path(self.h, int(path)), "qg_model_set_attention_path")
 

@@ -462,9 +462,15 @@ constexpr uint32_t kHeadWaves = 16;
 // ranges per head and with one.  Measured per layer against the split kernel
 // and its merge, whose time hardly depends on the length (us, whole step):
 // two ranges 56.8 / 58.7 at 500 positions and 59.0 / 58.6 at 700 (Qwen2-7B),
-// 55.0 / 55.7 and 57.3 / 55.7 (Llama-3-8B); one 28.5 / 29.9 at 200 and 32.1 /
-// 30.0 at 400 (Qwen2-0.5B).
-constexpr uint32_t kShortSeq = 512, kShortSeq1 = 256;
+// 55.0 / 55.7 and 57.3 / 55.7 (Llama-3-8B).  With one range the lines cross
+// later the larger the heads (four layers, one / split at 257, 320, 400 and 480
+// positions): head_dim 64 Q4_K of 14 heads 123.5 / 124.9, 126.9 / 125.2, 133 /
+// 125, 137 / 125, F16 of 32 heads 161 / 167, 164 / 167, 170.5 / 166.4, 173 / 166;
+// head_dim 128 Q4_K of 21 heads 176 / 185, 180 / 185, 187.5 / 185.5, 191 / 186,
+// F16 of 32 heads 334 / 338, 339 / 337, 348 / 336, 352 / 336; head_dim 256 F16
+// of 8 heads 175 / 196, 181 / 196, 189 / 196, 196 / 196.
+constexpr uint32_t kShortSeq = 512;
+constexpr uint32_t short_seq1(uint32_t hd) { return hd <= 64 ? 288 : hd <= 128 ? 320 : 480; }
 template <int E, int NR = 1>
 __global__ void __launch_bounds__(64 * kHeadWaves) attn_rope_head_k(AttnArgs a, float *__restrict__ out)
 {
@@ -1322,14 +1328,14 @@ bool two_range_ok(const qg_model *m)
 
 // the attention mode of the forward pass that writes cache slot `slot`: up to
 // kShortSeq cached positions whole heads as two position ranges per head
-// where every wo takes them (mode 2), else up to kShortSeq1 in one workgroup
+// where every wo takes them (mode 2), else up to short_seq1 in one workgroup
 // per head (mode 1); beyond, split over position ranges (mode 0).  att_path: 0 by length, 1
 // always one workgroup per head, 2 always split, 3 always two ranges where
 // the wo matrices allow it (else one workgroup per head).
 void pick_attention(qg_model *m, uint32_t slot)
 {
     const int whole = m->att_path != 1 && two_range_ok(m) ? 2 : 1;
-    const uint32_t most = whole == 2 ? qgm::kShortSeq : qgm::kShortSeq1;
+    const uint32_t most = whole == 2 ? qgm::kShortSeq : qgm::short_seq1(m->hd);
     const bool shrt = m->att_path == 1 || m->att_path == 3 || (m->att_path == 0 && slot + 1 <= most);
     m->att_mode = m->att_grp && shrt ? whole : 0;
 }

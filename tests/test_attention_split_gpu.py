@@ -49,3 +49,27 @@ def test_ranges_of_two_tiles(rinf, synth, oracle, ctx):
         dev.forward(i, n + i, logits)
         assert normwise_err(logits, ref.forward(i, n + i)) <= DEEP_TOL, i
     dev.close()
+
+
+@pytest.mark.parametrize("embed,heads,kv,mix,most", [(384, 6, 2, "q4_k_m", 288), (384, 3, 1, "q4_k_m", 320),
+                                                     (512, 2, 1, "f16", 480)])
+def test_where_the_split_begins(rinf, synth, oracle, ctx, embed, heads, kv, mix, most):
+    """A wo that takes no two ranges (rows of 1.5 blocks, F16): one workgroup per
+    head up to the length where the split is as fast, which grows with the head
+    size."""
+    cfg = dict(SMALL, embed_dim=embed, n_heads=heads, n_kv_heads=kv, n_layers=1)
+    dev, _, _ = build(rinf, synth, oracle, ctx, cfg, mix, 35, most + 8)
+    prompt = np.arange(most + 1) * 37 % cfg["vocab_size"]
+    got = {}
+    for path in (0, 1, 2):
+        dev.reset()
+        dev.prefill(prompt[:most - 1])
+        dev.set_attention_path(path)
+        for pos in (most - 1, most):
+            logits = np.zeros(cfg["vocab_size"], np.float32)
+            dev.forward(int(prompt[pos]), pos, logits)
+            got[path, pos + 1] = logits.tobytes()
+        dev.set_attention_path(0)
+    assert got[1, most] != got[2, most] and got[1, most + 1] != got[2, most + 1]
+    assert got[0, most] == got[1, most] and got[0, most + 1] == got[2, most + 1]
+    dev.close()
