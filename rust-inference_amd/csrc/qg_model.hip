@@ -244,9 +244,9 @@ template <int E>
 __global__ void __launch_bounds__(256) attn_rope_split_k(AttnArgs a)
 {
     constexpr uint32_t HD = 64 * E, KS = HD / 16u;
-    __shared__ float sacc[4][kMaxGroup][HD];
+    __shared__ __align__(16) float sacc[4][kMaxGroup][HD];
     __shared__ float sml[4][kMaxGroup][2];
-    __shared__ float sp[4][16][20];
+    __shared__ __align__(16) float sp[4][16][20];
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t c = lane & 15u, g = lane >> 4;
     const uint32_t grp = a.grp, split = blockIdx.x % a.nsplit, h0 = (blockIdx.x / a.nsplit) * grp;

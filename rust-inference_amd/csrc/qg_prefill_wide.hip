@@ -39,6 +39,10 @@ typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+// Q6_K's row groups are 210 bytes a block: their pieces and scales start at any
+// even address
+typedef uint32_t v4u_2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32_2 __attribute__((aligned(2)));
 
 __device__ __forceinline__ h2 as_h2(uint32_t u) { return __builtin_bit_cast(h2, u); }
 __device__ __forceinline__ uint32_t as_u(h2 h) { return __builtin_bit_cast(uint32_t, h); }
@@ -163,15 +167,15 @@ template <> struct Wt<T_Q5_K> {
 template <> struct Wt<T_Q6_K> {
     static constexpr int NB = 2;
     static constexpr bool KQ = false;
-    struct Raw { uint4 l, h; uint32_t sc; uint32_t d; };
+    struct Raw { v4u l, h; uint32_t sc; uint32_t d; };
     __device__ static uint32_t slot0(uint32_t kq) { return ((kq >> 1) << 2) | ((kq & 1u) << 1); }
     __device__ static constexpr uint32_t mx(uint32_t m) { return ((m >> 1) << 3) | (m & 1u); }
     __device__ static Raw load(const uint8_t *W, uint32_t cs, uint32_t v, uint32_t c, uint32_t kq, uint32_t ni)
     {
         const uint8_t *p = W + (size_t)cs * 32u;
         const uint32_t o = v + c * 32u + (kq & 1u) * 16u;
-        return Raw{*(const uint4 *)(p + (o + (kq >> 1) * ni * 16u)), *(const uint4 *)(p + (o + 32u * ni)),
-                   *(const uint32_t *)(W + (size_t)cs * 8u + (v + 48u * ni + (kq & 1u) * 4u + c * 8u)),
+        return Raw{*(const v4u_2 *)(p + (o + (kq >> 1) * ni * 16u)), *(const v4u_2 *)(p + (o + 32u * ni)),
+                   *(const u32_2 *)(W + (size_t)cs * 8u + (v + 48u * ni + (kq & 1u) * 4u + c * 8u)),
                    (uint32_t)*(const uint16_t *)(W + (size_t)(cs >> 1) * 2u + (v + 52u * ni + (c >> 1) * 2u))};
     }
     __device__ static Sc2 scale(const Raw &w, uint32_t n, uint32_t kq)
@@ -323,7 +327,7 @@ __global__ void __launch_bounds__(512) wide_gemm_k(Jobs jobs, uint32_t row_tiles
     using P = Wt<T>;
     constexpr bool Q8 = T == T_Q8_0;
     constexpr uint32_t BLK = ONE && !Q8 ? 2u : 1u;         // chunks per flush of D
-    extern __shared__ uint8_t lds[];
+    extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t j8 = blockIdx.x >> 3, tt0 = j8 % tok_tiles;
     uint32_t tile = (j8 / tok_tiles) * 8u + (blockIdx.x & 7u);
     if (tile >= row_tiles * slices) return;
@@ -728,7 +732,7 @@ __global__ void __launch_bounds__(256) wide_attention_k(const float *__restrict_
 {
     constexpr uint32_t LK = HD + 4u, LP = kAttPos + 4u, KS = HD / 16u, NT = HD / 16u;
     constexpr uint32_t LD = kAttPos * HD / 4u / 256u;      // float4 of K (and of V) per thread and tile
-    extern __shared__ float att[];
+    extern __shared__ __align__(16) float att[];
     float *ks = att, *vs = ks + kAttPos * LK;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, g = lane >> 4;
     const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -59,6 +59,8 @@ __device__ __forceinline__ uint32_t rd16(const uint8_t *p) { return (uint32_t)p[
 
 // 16 bytes from a 4-byte-aligned address (global_load_dwordx4)
 struct __attribute__((packed, aligned(4))) U4a { uint32_t a, b, c, d; };
+// ... at an even address (Q6_K's row groups are 210 bytes a block)
+struct __attribute__((packed, aligned(2))) U4h { uint32_t a, b, c, d; };
 
 // quant.rs:606-615 on the three scale dwords s0 (bytes 0-3), s1 (4-7), s2 (8-11)
 __device__ __forceinline__ void k4sm(uint32_t j, uint32_t s0, uint32_t s1, uint32_t s2,
@@ -549,7 +551,7 @@ __device__ __forceinline__ void unit_dot(const uint8_t *G, uint32_t ni, uint32_t
         }
     } else if constexpr (T == T_Q6_K) {
         const uint32_t it = 2u * c + (kq & 1u), pc = kq >> 1;
-        const U4a l4 = *(const U4a *)(G + (pc * ni + it) * 16u), h4 = *(const U4a *)(G + (2u * ni + it) * 16u);
+        const U4h l4 = *(const U4h *)(G + (pc * ni + it) * 16u), h4 = *(const U4h *)(G + (2u * ni + it) * 16u);
         const uint32_t sw = ldu32(G + 48u * ni + 4u * it) >> (8u * pc);
         const float d = h2f_exact(ldu16(G + 52u * ni + 2u * (c >> 1)));
         const float s0 = d * (float)(int8_t)sw, s1 = d * (float)(int8_t)(sw >> 16);
@@ -613,7 +615,7 @@ constexpr size_t unit_lds(uint32_t cols) { return 32u * (cols / 128u | 1u) * 16u
 template <uint32_t T>
 __global__ void __launch_bounds__(64 * kUnitWaves) gemv_units(QuadArgs a)
 {
-    extern __shared__ float ux[];
+    extern __shared__ __align__(16) float ux[];
     const uint32_t nchunk = a.cols / 128u, S = nchunk | 1u, lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (uint32_t i = threadIdx.x; i < a.cols / 4u; i += 64u * kUnitWaves)
