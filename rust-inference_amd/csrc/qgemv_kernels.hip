@@ -462,7 +462,8 @@ __global__ void __launch_bounds__(256) gemv_quads(QuadArgs a)
     auto add = [](float s, float p, float q) { return FUSE ? __builtin_fmaf(p, q, s) : s + p * q; };
     if constexpr (AL) {                                          // cols % 4 == 0: rows start on quads
 #pragma unroll 4
-        for (uint32_t c = 4u * tid; c < a.cols; c += 4u * TPR) {
+        for (uint32_t q = tid; q < a.cols / 4u; q += TPR) {      // (a counter of elements could wrap)
+            const uint32_t c = 4u * q;
             const f4 x = *(const f4u *)(a.x + c);
 #pragma unroll
             for (uint32_t i = 0; i < R; i++) {
@@ -477,19 +478,20 @@ __global__ void __launch_bounds__(256) gemv_quads(QuadArgs a)
             const uint32_t h = (uint32_t)f0[i] & 3u;             // elements of the first quad before the row
             // the whole quads inside the row, then (lanes 0 and 1) its first
             // and last quad where they are not
-            const uint32_t q0 = h ? 1u : 0u, q1 = (h + a.cols) / 4u;
+            const uint64_t end = (uint64_t)h + a.cols;
+            const uint32_t q0 = h ? 1u : 0u, q1 = (uint32_t)(end / 4u);
             const float *xr = a.x - h;
             const IX fa = f0[i] - h;
 #pragma unroll 4
             for (uint32_t q = q0 + tid; q < q1; q += TPR) {
                 const f4 x = *(const f4u *)(xr + 4u * q);
-                const f4 v = quad<T, RP>(base[i], a.ni, fa + 4u * q);
+                const f4 v = quad<T, RP>(base[i], a.ni, fa + (IX)4u * q);
 #pragma unroll
                 for (int j = 0; j < 4; j++) acc[i] = add(acc[i], v[j], x[j]);
             }
             const uint32_t q = tid == 0u ? 0u : q1;
-            if ((tid == 0u && h) || (tid == 1u && 4u * q1 < h + a.cols && (q1 > 0u || !h))) {
-                const f4 v = quad<T, RP>(base[i], a.ni, fa + 4u * q);
+            if ((tid == 0u && h) || (tid == 1u && (end & 3u) && (q1 > 0u || !h))) {
+                const f4 v = quad<T, RP>(base[i], a.ni, fa + (IX)4u * q);
 #pragma unroll
                 for (uint32_t j = 0; j < 4u; j++) {
                     const uint32_t c = 4u * q + j - h;           // wraps below the row

@@ -89,3 +89,25 @@ def test_wrapped_layout(rinf, synth, oracle, ctx, t):
     mat.dequant_host(out)
     assert np.array_equal(out, oracle.dequantize(raw, dtype, rows * cols)[:rows * cols])
     c.close()
+
+
+def test_longest_rows(rinf, ctx):
+    """A row of 2^32 - 100 columns: the step past its end does not wrap the
+    counters (the loops end), and the last columns are read."""
+    import torch
+    cols = 2 ** 32 - 100
+    nb = -(-cols // 32)
+    raw = np.zeros(18 * nb, np.uint8)
+    for b in (0, nb - 2, nb - 1):
+        raw[18 * b:18 * b + 2] = np.array([0.5], np.float16).view(np.uint8)
+        raw[18 * b + 2:18 * b + 18] = 0x99                   # every value 0.5
+    mat = ctx.upload(raw, rinf.TYPE_IDS["Q4_0"], 1, cols)
+    del raw
+    x = torch.zeros(cols, device="cuda")
+    x[0], x[40], x[cols - 1], x[cols - 5] = 1.0, 100.0, 2.0, 4.0
+    y = torch.zeros(1, device="cuda")
+    torch.cuda.synchronize()
+    mat.matvec_dev(x, y)
+    ctx.synchronize()
+    assert y.item() == 3.5
+    mat.free()
