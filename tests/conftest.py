@@ -56,3 +56,11 @@ def normwise_err(y, ref):
 # normwise: max|y - y_ref| / max|y_ref|; a per-element relative bound is
 # unattainable where outputs cancel to near zero).
 GEMV_TOL = 1e-4
+
+# The same for the kernels that split x into two pieces or a sum over ranges,
+# tight enough that a piece lost in part of a row shows: the oracle's own
+# sequential f32 sums of n terms are off by about sqrt(n) 2^-24 (4e-6 for the
+# longest rows here), a few matrices deep; measured 0.1e-6 to 7e-6.  x without
+# its low piece (f16 alone) is 2e-4 off in a mat-vec, 1e-4 with a quarter of the
+# columns so, 4e-5 with a sixteenth.
+TIGHT_TOL = 2e-5

@@ -3,14 +3,14 @@ oracle where its tiles and ranges end: 1 to 65 cached positions (a wave of 16
 with none, one and all of its positions, the second tile of 64), 4100 (ranges
 of two tiles), grouped heads of every size up to 8 and one, head_dim 64, 128
 and 256.  The prompt goes through the token-by-token path up to 70 positions,
-so every length is checked; DEEP_TOL (1e-4 normwise)."""
+so every length is checked; TIGHT_TOL (2e-5 normwise)."""
 from __future__ import annotations
 
 import numpy as np
 import pytest
 
-from conftest import normwise_err
-from test_decode_gpu import DEEP_TOL, SMALL, build
+from conftest import TIGHT_TOL, normwise_err
+from test_decode_gpu import SMALL, build
 
 pytestmark = pytest.mark.gpu
 
@@ -24,7 +24,7 @@ def test_every_length(rinf, synth, oracle, ctx, embed, heads, kv):
     for pos in range(70):
         tok = (pos * 37 + 5) % cfg["vocab_size"]
         dev.forward(tok, pos, logits)
-        assert normwise_err(logits, ref.forward(tok, pos)) <= DEEP_TOL, pos
+        assert normwise_err(logits, ref.forward(tok, pos)) <= TIGHT_TOL, pos
     # a shorter conversation over the same cache: rows past it hold old values
     dev.reset()
     dev2, ref2, _ = build(rinf, synth, oracle, ctx, cfg, "q8_0", 31, 80)
@@ -32,7 +32,7 @@ def test_every_length(rinf, synth, oracle, ctx, embed, heads, kv):
     for pos in range(5):
         tok = (pos * 91 + 1) % cfg["vocab_size"]
         dev.forward(tok, pos, logits)
-        assert normwise_err(logits, ref2.forward(tok, pos)) <= DEEP_TOL, pos
+        assert normwise_err(logits, ref2.forward(tok, pos)) <= TIGHT_TOL, pos
     dev.close()
 
 
@@ -47,7 +47,7 @@ def test_ranges_of_two_tiles(rinf, synth, oracle, ctx):
     logits = np.zeros(300, np.float32)
     for i in range(30):
         dev.forward(i, n + i, logits)
-        assert normwise_err(logits, ref.forward(i, n + i)) <= DEEP_TOL, i
+        assert normwise_err(logits, ref.forward(i, n + i)) <= TIGHT_TOL, i
     dev.close()
 
 

@@ -6,11 +6,14 @@ f32 accumulation).  Checked against the oracle's token-by-token
 forward pass (oracle/qref_model.c, transformer.rs:63-98 as model.rs:361-365
 calls it): the last prompt token's logits, then greedy decode steps on the
 caches the prefill wrote (every cached position's K/V enters those steps),
-within DEEP_TOL, identical tokens.  Also: chunks of 64 tokens, a prefill that
-continues a cache, the token-by-token fallback for a mix without an MFMA
-path (F16), generate with the batched prefill, and layer matrices wrapped
-in the GGUF layout (qg_wrap_device) so that the GEMM's GGUF-layout loaders
-run: rows straddling superblocks (cols = 896) and whole-block rows."""
+within DEEP_TOL, identical tokens.  Calls of at most 64 tokens (and longer
+prompts over GGUF-layout matrices) run the 64-token chunks' kernels of
+qg_prefill.hip, longer ones those of qg_prefill_wide.hip.  Also: chunks of 64
+tokens, a prefill that continues a cache, the token-by-token fallback for a
+mix without an MFMA path (F16), generate with the batched prefill, and layer
+matrices wrapped in the GGUF layout (qg_wrap_device) so that the GEMM's
+GGUF-layout loaders run: rows straddling superblocks (cols = 896) and
+whole-block rows."""
 from __future__ import annotations
 
 import numpy as np
@@ -47,8 +50,8 @@ def prefill_and_compare(rinf, synth, oracle, ctx, cfg, mix, seed, n_prompt, n_ne
     dev, ref, shared = build(rinf, synth, oracle, ctx, cfg, mix, seed, max_seq)
     prompt = np.random.default_rng(seed).integers(0, cfg["vocab_size"], n_prompt)
     logits = np.zeros(cfg["vocab_size"], np.float32)
-    parts = [prompt] if split is None else [prompt[:split], prompt[split:]]
-    for p in parts:
+    at = [] if split is None else list(np.atleast_1d(split))      # where the calls' parts begin
+    for p in np.split(prompt, at):
         dev.prefill(p, logits)
     ref_l = None
     for pos, tok in enumerate(prompt):
@@ -69,11 +72,12 @@ def test_small_model_prefill(rinf, synth, oracle, ctx, mix):
     assert e0 <= DEEP_TOL and max(errs) <= DEEP_TOL
 
 
-def test_prefill_chunks_and_continuation(rinf, synth, oracle, ctx):
-    """150 prompt tokens (chunks of 64, 64, 22), fed as 37 + 113 (the second
-    call continues the caches at position 37)."""
+@pytest.mark.parametrize("split", [37, (37, 101), (64, 128)], ids=["37-113", "37-64-49", "64-64-22"])
+def test_prefill_chunks_and_continuation(rinf, synth, oracle, ctx, split):
+    """150 prompt tokens in two or three calls, each continuing the caches: one of
+    113 tokens (a wide chunk), or 64-token chunks only."""
     cfg = dict(SMALL, n_layers=2)
-    e0, errs, out = prefill_and_compare(rinf, synth, oracle, ctx, cfg, "q4_k_m", 43, 150, 6, 200, split=37)
+    e0, errs, out = prefill_and_compare(rinf, synth, oracle, ctx, cfg, "q4_k_m", 43, 150, 6, 200, split=split)
     print(f"chunks: prefill logits err {e0:.2e}, decode max {max(errs):.2e}", flush=True)
     assert e0 <= DEEP_TOL and max(errs) <= DEEP_TOL
 
@@ -88,15 +92,16 @@ def test_qwen2_7b_layer_shape_prefill(rinf, synth, oracle, ctx, mix):
     assert e0 <= DEEP_TOL and max(errs) <= DEEP_TOL
 
 
+@pytest.mark.parametrize("n,split", [(100, 30), (100, 60), (150, (64, 128))], ids=["30-70", "60-40", "64-64-22"])
 @pytest.mark.parametrize("hd", [64, 128, 256])
-def test_prefill_attention_head_dims(rinf, synth, oracle, ctx, hd):
-    """The prefill attention (f32 MFMA, tiles of 64 cached positions) at
-    head_dim 64, 128 and 256, two query heads per kv head: 100 prompt tokens
-    fed as 30 + 70 (the second call continues the caches; up to 100
-    positions, two tiles), then greedy steps."""
+def test_prefill_attention_head_dims(rinf, synth, oracle, ctx, hd, n, split):
+    """The prefill attention (f32 MFMA) at head_dim 64, 128 and 256, two query
+    heads per kv head: calls that continue the caches, 70 tokens through the
+    wide chunks' kernel, or 64 and fewer through pf_attention_k with two and
+    three of its tiles of 64 cached positions; then greedy steps."""
     heads = 1024 // hd
     cfg = dict(SMALL, n_layers=1, embed_dim=1024, n_heads=heads, n_kv_heads=max(1, heads // 2), hidden_dim=512)
-    e0, errs, out = prefill_and_compare(rinf, synth, oracle, ctx, cfg, "q4_k_m", 53, 100, 4, 128, split=30)
+    e0, errs, out = prefill_and_compare(rinf, synth, oracle, ctx, cfg, "q4_k_m", 53, n, 4, 192, split=split)
     print(f"head_dim {hd}: prefill logits err {e0:.2e}, decode max {max(errs):.2e}", flush=True)
     assert e0 <= DEEP_TOL and max(errs) <= DEEP_TOL
 
@@ -197,19 +202,20 @@ def build_wrapped(rinf, synth, oracle, ctx, cfg, mix, seed, max_seq):
     return dev, ref, keep, layouts
 
 
+@pytest.mark.parametrize("n", [40, 150])
 @pytest.mark.parametrize("embed,hidden,mix", [(896, 1024, "q4_k_m"), (3584, 1024, "q4_k_m"), (3584, 1024, "q8_0")],
                          ids=["straddle-896", "whole-3584", "q8_0-3584"])
-def test_prefill_gguf_layout_matrices(rinf, synth, oracle, ctx, embed, hidden, mix):
+def test_prefill_gguf_layout_matrices(rinf, synth, oracle, ctx, embed, hidden, mix, n):
     """Wrapped (GGUF-layout) layer matrices through the batched prefill:
     Q4_K rows of 896 columns straddle superblocks (the general loader), Q4_K,
     Q6_K and Q8_0 rows of 3584 / 1024 columns hold whole blocks (the
-    whole-block loader); 2 layers, a 40-token prompt, then 6 greedy steps,
-    against the oracle."""
+    whole-block loader); 2 layers, a prompt of 40 tokens or of three 64-token
+    chunks, then 6 greedy steps, against the oracle."""
     heads = embed // 64 if embed == 896 else 28
     cfg = dict(SMALL, n_layers=2, embed_dim=embed, n_heads=heads, n_kv_heads=2 if embed == 896 else 4,
                hidden_dim=hidden)
-    dev, ref, keep, layouts = build_wrapped(rinf, synth, oracle, ctx, cfg, mix, 83, 64)
-    prompt = np.random.default_rng(83).integers(0, cfg["vocab_size"], 40)
+    dev, ref, keep, layouts = build_wrapped(rinf, synth, oracle, ctx, cfg, mix, 83, n + 24)
+    prompt = np.random.default_rng(83).integers(0, cfg["vocab_size"], n)
     logits = np.zeros(cfg["vocab_size"], np.float32)
     dev.prefill(prompt, logits)
     ref_l = None
