@@ -30,8 +30,8 @@ struct qg_mat {
     qg::Plan plan;     // plan.rp: the stream kernels read d_rp
 };
 
-// The bytes the stream GEMV kernels read (the dequant and generic kernels
-// read the GGUF layout: d, or qg_mat_gguf).
+// The bytes the GEMV and whole-matrix dequant kernels read (single rows and
+// stacking read the GGUF layout: d, or qg_mat_gguf).
 inline const uint8_t *qg_gemv_bytes(const qg_mat *m) { return m->plan.rp ? m->d_rp : m->d; }
 
 // Device bytes of the matrix (both layouts it holds, tail pads included).

@@ -296,12 +296,16 @@ struct Jobs {
 // of 128 elements of x (64 KB) are copied straight to LDS, two buffers in
 // turn; a wave's weights go to registers one chunk ahead.
 //
-// What bounds it: the CU's issue.  A chunk of Q4_K is 136 MFMAs of 16 cycles
-// per wave, two waves to a SIMD (4352 cycles), and 130 LDS reads; it takes
-// about 9400 cycles (gate and up of Llama-3-8B over 1001 tokens, Q4_K: 562 us,
-// 856 TFLOP/s of f16 products), without the copies and weight loads 30 % less
-// and without the decode 25 % less.  Measured against it (Q5_K gate and up /
-// Q6_K down, us): this shape 610 / 327; wave tiles of 64 tokens x 48 rows 666
+// What bounds it: two waves a SIMD that issue or wait together.  A chunk of
+// Q4_K or Q5_K is 136 MFMAs of 16 cycles per wave, two waves to a SIMD (4352
+// cycles), and 72 LDS reads; gate and up of Llama-3-8B over 1001 tokens in Q5_K
+// (526-555 us, 3.5 tiles a CU in 4 rounds) take about 8500 cycles a chunk.  Of
+// its wave cycles 30 % issue, 32 % wait to issue and 38 % wait for data and at
+// the barriers; the matrix cores are busy in 45 % of all SIMD cycles (Q6_K down:
+// 68 %), the LDS in 25 % of the CUs'.  Without the copies and weight
+// loads a chunk took 30 % less, without the decode 25 % less.  Measured against
+// it, with three products of Q6_K (Q5_K gate and up / Q6_K down, us): this shape
+// 610 / 327; wave tiles of 64 tokens x 48 rows 666
 // / 437, of 64 x 64 1221 / 914 (registers spill); four waves of 128 x 64, one
 // to a SIMD, 820 / 410; copies and loads all requested at the start of a
 // chunk instead of between its steps 734 / 590 (64 x 48: the memory pipe's
@@ -584,7 +588,8 @@ __device__ __forceinline__ void sum8(const float *p, uint32_t ns, uint64_t sstri
 // position j ^ (t & 15) of the token's 256 bytes, the sums of xs per 32
 // elements (two f16 pieces) and 2^-e_g (NaN when the group's x is not finite),
 // of each of the group's chunks.  32 threads hold a group.  a, b: sums of na,
-// nb slices.  PM: 8-element pieces per thread (n <= 4096 PM).
+// nb slices.  PM: 8-element pieces per thread (n <= 4096 PM); instances of 1, 2,
+// 5 and 8, so rows of 14336 (3.5 pieces) and 18944 (4.6) share one.
 template <int PM>
 __global__ void __launch_bounds__(512) wide_planes_k(const float *__restrict__ a, uint32_t na, const float *__restrict__ b,
                                                      uint32_t nb, uint64_t sstride, float *__restrict__ sum_out,

@@ -98,8 +98,10 @@ int grow_device(qg_ctx *ctx, float **p, size_t *cap, size_t n)
 }
 
 // vectors of qg_matvec_host up to this length cross by a kernel (measured, us
-// per call, kernel / copy commands: Q8_0 896 x 896 20.8 / 21.3, Q6_K 3584 x
-// 18944 32.2 / 37.4, Q4_K 18944 x 3584 30.0 / 38.1, Q8_0 1024 x 65536 59 / 378)
+// per call, kernel / copy commands: Q8_0 896 x 896 21.1 / 21.3, Q6_K 3584 x
+// 18944 32.2 / 37.4, Q4_K 18944 x 3584 30.0 / 38.1; Q8_0 of 64 columns and 2^16,
+// 2^18, 2^20 rows 35 / 42, 85 / 92, 272 / 277; of 64 rows and as many columns 57
+// / 70, 176 / 225, 657 / 802).  Beyond it nothing is measured.
 constexpr size_t kCopyFloats = 1u << 20;
 
 int new_mat(qg_ctx *ctx, uint8_t *d, size_t nbytes, uint32_t type, size_t rows, size_t cols,
@@ -121,9 +123,10 @@ int new_mat(qg_ctx *ctx, uint8_t *d, size_t nbytes, uint32_t type, size_t rows, 
     }
     // Owned Q8_0 / Q4_K / Q5_K / Q6_K matrices are kept in the repacked layout
     // the stream kernels read with contiguous loads (the same bytes -- for
-    // Q5_K the same bits -- rearranged), and only in it: d is freed, and the
-    // dequant kernels get the GGUF layout back from qg_mat_gguf.  Bytes
-    // wrapped from caller memory keep the GGUF-layout kernels.
+    // Q5_K the same bits -- rearranged), and only in it: d is freed, and what
+    // needs the GGUF layout gets it back from qg_mat_gguf (one row, stacking;
+    // the dequant kernels read either).  Bytes wrapped from caller memory keep
+    // the GGUF-layout kernels.
     if (owned && qg::repack_eligible(type, m->plan, rows)) {
         uint8_t *r = nullptr;
         hipError_t e = qg_alloc_injected(ctx) ? hipErrorOutOfMemory : hipMalloc((void **)&r, nbytes + qg::kTailPad);

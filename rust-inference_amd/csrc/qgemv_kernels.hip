@@ -3185,8 +3185,8 @@ int launch_gemv_norm_pair(uint32_t t1, const Plan &p1, const uint8_t *w1, size_t
     uint32_t per1 = p1.per_team ? p1.per_team : 1u, per2 = p2.per_team ? p2.per_team : 1u;
     // Small parts run in smaller workgroups, one team batch each, on as many
     // CUs as there are, where a thread still holds its share of x in
-    // registers (two 16-element pieces): Qwen2-0.5B's [Q;K] and V, 18 + 4
-    // workgroups of 512 threads in 6.2 us, are 144 + 32 of 64 in 4.4
+    // registers (two 16-element pieces): Qwen2-0.5B's [Q;K] and V, 16 + 4
+    // workgroups of 512 threads in 5.8 us, are 128 + 32 of 64 in 4.1
     uint32_t block = kPairBlock;
     for (uint32_t b : {64u, 128u, 256u})
         if (per1 == 1u && per2 == 1u && b % p1.ts == 0 && b % p2.ts == 0 && cols <= 32u * b &&
