@@ -1787,15 +1787,22 @@ int qg_model_create(qg_ctx *ctx, const qg_model_config *cfg, qg_model **out)
     m->kv_dim = n_kv * hd;
     m->n_rep = c.n_heads / n_kv;
     // attention layout: workgroups of grp query heads (a divisor of n_rep, at
-    // most 8) times up to 64 position ranges of whole tiles of 64 positions;
-    // any max_seq_len
+    // most 8) times up to 64 position ranges of whole tiles of 64 positions,
+    // about one workgroup per CU in all at long sequences: with more, the CUs
+    // take them in turns (us a step of two layers, head_dim 128: 32 groups at
+    // 520 / 2000 / 8000 positions 87 / 101 / 165 with 8 ranges, 112 / 125 / 204
+    // with 32, 115 / 126 / 222 with 64; 8 groups 77 / 78 / 93 with 32, 79 / 80 /
+    // 104 with 64, 77 / 81 / 105 with 16; 4 groups 76 / 76 / 81 with 64, 77 / 77
+    // / 87 with 32).  At least 2, for the two ranges of attn_rope_head_k.  Any
+    // max_seq_len
     constexpr size_t kLdsMax = 65536;
     if (hd == 64 || hd == 128 || hd == 256) {
         uint32_t grp = 1;
         for (uint32_t d = 1; d <= qgm::kMaxGroup; d++)
             if (m->n_rep % d == 0) grp = d;
+        const uint32_t groups = c.n_heads / grp, cus = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
         m->att_grp = grp;
-        m->att_nsplit = qgm::kMaxSplit;
+        m->att_nsplit = std::min(std::max((cus + groups - 1) / groups, 2u), qgm::kMaxSplit);
     } else {
         m->att_lds = ((size_t)hd + c.max_seq_len) * sizeof(float);
         if (m->att_lds > kLdsMax) {

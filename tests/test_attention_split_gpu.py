@@ -73,3 +73,20 @@ def test_where_the_split_begins(rinf, synth, oracle, ctx, embed, heads, kv, mix,
     assert got[1, most] != got[2, most] and got[1, most + 1] != got[2, most + 1]
     assert got[0, most] == got[1, most] and got[0, most + 1] == got[2, most + 1]
     dev.close()
+
+
+def test_ranges_of_many_groups(rinf, synth, oracle, ctx):
+    """One workgroup per head and kv head, 16 of them: 16 ranges each, of two tiles
+    beyond 1024 positions."""
+    cfg = dict(SMALL, embed_dim=1024, n_heads=16, n_kv_heads=16, hidden_dim=256, n_layers=1, vocab_size=300)
+    n = 1020
+    dev, ref, _ = build(rinf, synth, oracle, ctx, cfg, "q8_0", 34, n + 40)
+    prompt = np.random.default_rng(6).integers(0, 300, n)
+    dev.prefill(prompt)
+    for pos, tok in enumerate(prompt):
+        ref.forward(int(tok), pos)
+    logits = np.zeros(300, np.float32)
+    for i in range(30):
+        dev.forward(i, n + i, logits)
+        assert normwise_err(logits, ref.forward(i, n + i)) <= TIGHT_TOL, i
+    dev.close()
