@@ -15,7 +15,8 @@
 // attention softmax is split over position ranges):
 //   RMSNorm          math.rs:237-257 (RmsNorm::forward), inside the next GEMV
 //                    with the residual add of transformer.rs:31-46
-//   attn_rope_split_k  attention.rs:66-121 for head_dim 64/128/256: bias
+//   attn_rope_split_k, attn_rope_split_vec_k
+//                    attention.rs:66-121 for head_dim 64/128/256: bias
 //                    add, RoPE on q and k (rope.rs:88-96, pairs 2i/2i+1), KV
 //   attn_combine_k   append (kv_cache.rs:52-73), then attention over one range
 //                    of positions for the query heads of one kv head; then the
@@ -49,10 +50,16 @@ constexpr uint32_t kMaxGroup = 8;         // query heads per attention workgroup
 constexpr uint32_t kMaxSplit = 64;        // position ranges per head
 constexpr uint32_t kRangeTile = 64;       // positions a workgroup takes at a time (16 per wave)
 
-// Positions per range for seq cached positions (whole tiles; the last range
-// may hold fewer); ranges = ceil(seq / len) <= nsplit.
-__host__ __device__ __forceinline__ uint32_t range_len(uint32_t seq, uint32_t nsplit)
+constexpr uint32_t kMinLen = 8;           // ... at least, in attn_rope_split_vec_k
+
+// Positions per range for seq cached positions (whole tiles, or with vec any
+// number; the last range may hold fewer); ranges = ceil(seq / len) <= nsplit.
+__host__ __device__ __forceinline__ uint32_t range_len(uint32_t seq, uint32_t nsplit, bool vec)
 {
+    if (vec) {
+        const uint32_t l = (seq + nsplit - 1) / nsplit;
+        return l > kMinLen ? l : kMinLen;
+    }
     const uint32_t t = (seq + kRangeTile - 1) / kRangeTile;
     return (t + nsplit - 1) / nsplit * kRangeTile;
 }
@@ -263,7 +270,7 @@ __global__ void __launch_bounds__(256) attn_rope_split_k(AttnArgs a)
     for (int b = 0; b < E; b++)
         vn[b] = *(const v4f *)(a.v + kvo + 64u * b + 4u * c) + *(const v4f *)(a.bv + kvo + 64u * b + 4u * c);
     const uint32_t pos = a.st->pos, slot = a.st->slot, seq = slot + 1;
-    const uint32_t len = range_len(seq, a.nsplit), j0 = split * len, j1 = min(seq, j0 + len);
+    const uint32_t len = range_len(seq, a.nsplit, false), j0 = split * len, j1 = min(seq, j0 + len);
     if (j0 >= seq) return;
     // K and V rows of the 16 positions at base, clamped into the rows that exist
     v4f kk[KS], vv[4][E];
@@ -395,18 +402,208 @@ __global__ void __launch_bounds__(256) attn_rope_split_k(AttnArgs a)
     }
 }
 
-// out[h] = sum_s w_s part_s with w_s = exp(m_s - max m) / sum_s exp(m_s - max m) l_s:
-// the softmax-weighted sum of v over all positions.  One workgroup of 1024
-// threads per head: wave w takes dimensions 64 (w % E) .. of the ranges s = w / E
-// (mod 16 / E), all of them requested at once (clamped to the ranges in use;
-// those need the step record only for their number), and derives the ranges'
-// weights itself, one per lane.
+// The same on the vector units: where a workgroup has few heads (and with
+// head_dim 256, whose tile on the matrix cores takes all 512 registers) one
+// position and head at a time starts sooner.  Workgroup (head group, range): 4
+// waves, each lane owns dimensions lane + 64 e (every K and V row is one
+// coalesced read shared by the group's heads).  A wave takes positions j0 + wave
+// + 4 p in chunks of kPW, all K and V rows of a chunk loaded before any use,
+// with a running (max, sum, output) per head (the softmax of attention.rs:101-119
+// over the wave's positions); the four waves are merged in LDS.  Same outputs as
+// attn_rope_split_k.
+// Positions per wave per chunk: the chunk's code is unrolled over heads and
+// positions, and a larger chunk made the kernel slower (straight-line code
+// fetched cold by every workgroup) while short ranges fill only one chunk.
+constexpr uint32_t kPW = 2;
 template <int E>
-__global__ void __launch_bounds__(1024) attn_combine_k(const float *__restrict__ part, const float *__restrict__ ml,
-                                                       float *__restrict__ out, const Step *__restrict__ st,
-                                                       uint32_t nsplit)
+__global__ void __launch_bounds__(256) attn_rope_split_vec_k(AttnArgs a)
 {
-    constexpr uint32_t HD = 64 * E, NW = 16u / E, PER = kMaxSplit / NW;
+    constexpr uint32_t HD = 64 * E;
+    __shared__ float sacc[4][kMaxGroup][HD];
+    __shared__ float sml[4][kMaxGroup][2];
+    // wave index as a uniform value: the position loop's bounds depend on it,
+    // and a per-lane value would turn every branch on them into exec masking
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t grp = a.grp, split = blockIdx.x % a.nsplit, h0 = (blockIdx.x / a.nsplit) * grp;
+    const uint32_t kvo = (h0 / a.n_rep) * HD;
+    // Every load below is unconditional (clamped indices, selects after the
+    // loads): a load behind a branch waits for everything issued before it.
+    // The projections do not depend on the step record, so they are in flight
+    // while it arrives.
+    float qv[kMaxGroup][E], kn[E], vn[E];
+#pragma unroll
+    for (uint32_t r = 0; r < kMaxGroup; r++)
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const uint32_t i = (h0 + (r < grp ? r : 0u)) * HD + lane + 64 * e;
+            qv[r][e] = a.q[i] + a.bq[i];
+        }
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        kn[e] = a.k[kvo + lane + 64 * e] + a.bk[kvo + lane + 64 * e];
+        vn[e] = a.v[kvo + lane + 64 * e] + a.bv[kvo + lane + 64 * e];
+    }
+    const uint32_t pos = a.st->pos, slot = a.st->slot, seq = slot + 1;
+    const uint32_t len = range_len(seq, a.nsplit, true);
+    const uint32_t j0 = split * len, j1 = min(seq, j0 + len);
+    // K and V rows of this wave's positions j0 + wave + 4 p, kPW at a time,
+    // clamped into the cache rows that exist (a workgroup past seq loads and
+    // exits); the next chunk is in flight while one is used
+    float kk[kPW][E], vv[kPW][E], nk[kPW][E], nv[kPW][E];
+    auto load = [&](uint32_t b, float (&ko)[kPW][E], float (&vo)[kPW][E]) {
+#pragma unroll
+        for (uint32_t p = 0; p < kPW; p++) {
+            const uint32_t j = min(b + 4 * p, slot);
+            const float *kr = a.kc + (size_t)j * a.kv_dim + kvo, *vr = a.vc + (size_t)j * a.kv_dim + kvo;
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                ko[p][e] = kr[lane + 64 * e];
+                vo[p][e] = vr[lane + 64 * e];
+            }
+        }
+    };
+    uint32_t base = j0 + wave;
+    load(base, kk, vv);
+    // cos / sin of this lane's pairs (the table rows of `pos`)
+    float cv[E], sv[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        cv[e] = a.cos_t[(size_t)pos * (HD / 2) + ((lane + 64 * e) >> 1)];
+        sv[e] = a.sin_t[(size_t)pos * (HD / 2) + ((lane + 64 * e) >> 1)];
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kMaxGroup; r++)
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const float o = __shfl_xor(qv[r][e], 1, 64);
+            qv[r][e] = r < grp ? rope1(qv[r][e], o, lane + 64 * e, cv[e], sv[e]) : 0.f;
+        }
+#pragma unroll
+    for (int e = 0; e < E; e++) kn[e] = rope1(kn[e], __shfl_xor(kn[e], 1, 64), lane + 64 * e, cv[e], sv[e]);
+    if (j0 >= seq) return;
+    const bool has_new = j1 == seq;
+    if (has_new && h0 % a.n_rep == 0 && wave == 0) {
+        float *kr = a.kc + (size_t)slot * a.kv_dim + kvo, *vr = a.vc + (size_t)slot * a.kv_dim + kvo;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            kr[lane + 64 * e] = kn[e];
+            vr[lane + 64 * e] = vn[e];
+        }
+    }
+    float m[kMaxGroup], l[kMaxGroup], acc[kMaxGroup][E];
+#pragma unroll
+    for (uint32_t r = 0; r < kMaxGroup; r++) {
+        m[r] = -INFINITY;
+        l[r] = 0.f;
+#pragma unroll
+        for (int e = 0; e < E; e++) acc[r][e] = 0.f;
+    }
+    for (; base < j1; base += 4 * kPW) {
+        const uint32_t np = min((j1 - base + 3) / 4, kPW);   // this wave's positions in the chunk
+        if (base + 4 * kPW < j1) load(base + 4 * kPW, nk, nv);
+        // the slot being appended comes from registers (its cache row is written above)
+#pragma unroll
+        for (uint32_t p = 0; p < kPW; p++)
+            if (base + 4 * p == slot)
+#pragma unroll
+                for (int e = 0; e < E; e++) { kk[p][e] = kn[e]; vv[p][e] = vn[e]; }
+#pragma unroll
+        for (uint32_t r = 0; r < kMaxGroup; r++) {
+            if (r >= grp) break;
+            float sc[kPW], cm = -INFINITY;
+#pragma unroll
+            for (uint32_t p = 0; p < kPW; p++) {
+                if (p >= np) break;
+                float t = 0.f;
+#pragma unroll
+                for (int e = 0; e < E; e++) t += qv[r][e] * kk[p][e];
+                sc[p] = wave_sum(t) * a.scale;
+                cm = fmaxf(cm, sc[p]);
+            }
+            const float mn = fmaxf(m[r], cm);
+            const float al = m[r] == -INFINITY ? 0.f : expf(m[r] - mn);
+            float ls = 0.f, o[E];
+#pragma unroll
+            for (int e = 0; e < E; e++) o[e] = 0.f;
+#pragma unroll
+            for (uint32_t p = 0; p < kPW; p++) {
+                if (p >= np) break;
+                const float ex = expf(sc[p] - mn);
+                ls += ex;
+#pragma unroll
+                for (int e = 0; e < E; e++) o[e] += ex * vv[p][e];
+            }
+            l[r] = l[r] * al + ls;
+#pragma unroll
+            for (int e = 0; e < E; e++) acc[r][e] = acc[r][e] * al + o[e];
+            m[r] = mn;
+        }
+#pragma unroll
+        for (uint32_t p = 0; p < kPW; p++)
+#pragma unroll
+            for (int e = 0; e < E; e++) { kk[p][e] = nk[p][e]; vv[p][e] = nv[p][e]; }
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kMaxGroup; r++) {
+        if (r >= grp) break;
+#pragma unroll
+        for (int e = 0; e < E; e++) sacc[wave][r][lane + 64 * e] = acc[r][e];
+        if (lane == 0) { sml[wave][r][0] = m[r]; sml[wave][r][1] = l[r]; }
+    }
+    __syncthreads();
+    // merge the waves: weights exp(m_w - M) (0 for a wave without positions)
+    for (uint32_t i = threadIdx.x; i < grp * HD; i += blockDim.x) {
+        const uint32_t r = i / HD, d = i % HD;
+        float mx = sml[0][r][0];
+#pragma unroll
+        for (int w = 1; w < 4; w++) mx = fmaxf(mx, sml[w][r][0]);
+        float sum = 0.f, lsum = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const float mw = sml[w][r][0];
+            const float f = mw == -INFINITY ? 0.f : expf(mw - mx);
+            sum += f * sacc[w][r][d];
+            lsum += f * sml[w][r][1];
+        }
+        const size_t o = (size_t)(h0 + r) * a.nsplit + split;
+        a.part[o * HD + d] = sum;
+        if (d == 0) {
+            a.ml[2 * o] = mx;
+            a.ml[2 * o + 1] = lsum;
+        }
+    }
+}
+
+// Cached positions up to which attn_rope_split_vec_k is the faster of the two
+// (us a step of two layers, vec / matrix cores at 520, 1300, 2500 and 4000
+// positions): head_dim 256 in groups of one head 66 / 78, 68 / 78, 73 / 88, 80 /
+// 93 (8 heads; still 110 / 116 at 8000); of two 65 / 77, 67 / 77, 70 / 76, 75 / 79
+// (8 heads); of four 79 / 91, 83 / 92, 89 / 91, 98 / 94 (16); of eight 86 / 94, 93.5
+// / 94.0, 104 / 94, 121 / 94 (16); head_dim 128 in groups of one 83.5 / 86.0 at
+// 520, 85.3 / 86.3 at 700 and 88.5 / 86.4 at 900 (32 heads), 63 / 65, 67.3 / 68.5 at
+// 1300 and 75 / 74 at 2500 (16).  Larger groups of 128 and head_dim 64: the matrix
+// cores at every length.
+constexpr uint32_t vec_seq(uint32_t hd, uint32_t grp)
+{
+    if (hd == 256) return grp == 1 ? 0xFFFFFFFFu : grp == 2 ? 6144 : grp <= 4 ? 2560 : 1280;
+    return hd == 128 && grp == 1 ? 832 : 0;
+}
+
+// out[h] = sum_s w_s part_s with w_s = exp(m_s - max m) / sum_s exp(m_s - max m) l_s:
+// the softmax-weighted sum of v over all positions.  One workgroup of W waves
+// per head: wave w takes dimensions 64 (w % E) .. of the ranges s = w / E (mod
+// W / E), all of them requested at once (clamped to the ranges there are; those
+// in use need the step record only for their number), and derives the ranges'
+// weights itself, one per lane.  W = 16, or 4 for at most kFewSplit ranges (a
+// step of two layers at 520 positions, us: 16 heads of 256 with 16 ranges 84.7 ->
+// 81.6).
+constexpr uint32_t kFewSplit = 16;
+template <int E, int W, bool VEC>
+__global__ void __launch_bounds__(64 * W) attn_combine_k(const float *__restrict__ part, const float *__restrict__ ml,
+                                                         float *__restrict__ out, const Step *__restrict__ st,
+                                                         uint32_t nsplit)
+{
+    constexpr uint32_t HD = 64 * E, NW = W / E, PER = (W == 16 ? kMaxSplit : kFewSplit) / NW;
     __shared__ float red[NW][HD];
     const uint32_t h = blockIdx.x, lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t d = 64u * (wave % E) + lane, s0 = wave / E;
@@ -415,7 +612,7 @@ __global__ void __launch_bounds__(1024) attn_combine_k(const float *__restrict__
     float u[PER];
 #pragma unroll
     for (uint32_t i = 0; i < PER; i++) u[i] = p[(size_t)min(s0 + i * NW, nsplit - 1u) * HD];
-    const uint32_t seq = st->slot + 1, len = range_len(seq, nsplit), nr = (seq + len - 1) / len;
+    const uint32_t seq = st->slot + 1, len = range_len(seq, nsplit, VEC), nr = (seq + len - 1) / len;
     const float ms = lane < nr ? v.x : -INFINITY;
     const float mx = wave_max(ms);
     const float w = lane < nr ? expf(ms - mx) : 0.f;
@@ -862,10 +1059,10 @@ struct qg_model {
     // captured graphs per attention mode: [0] the split attention
     // (attn_rope_split_k + attn_combine_k), [1] whole heads in one workgroup
     // each (attn_rope_head_k), [2] two position ranges per head merged in the
-    // wo GEMV's input (attn_rope_head_k<E, 2> + launch_gemv_attn); att_mode
-    // selects what enqueue_forward launches
-    hipGraphExec_t g_fwd[3] = {nullptr, nullptr, nullptr};   // forward pass
-    hipGraphExec_t g_dec[3] = {nullptr, nullptr, nullptr};   // sample + advance + forward (generate)
+    // wo GEMV's input (attn_rope_head_k<E, 2> + launch_gemv_attn), [3] as [0]
+    // with attn_rope_split_vec_k; att_mode selects what enqueue_forward launches
+    hipGraphExec_t g_fwd[4] = {};         // forward pass
+    hipGraphExec_t g_dec[4] = {};         // sample + advance + forward (generate)
     int att_mode = 0;
     int att_path = 0;                     // qg_model_set_attention_path
     float g_dec_penalty = 0.f;
@@ -926,7 +1123,7 @@ hipError_t copy_wait(qg_model *m, void *dst, const void *src, size_t n, hipMemcp
 
 void drop_graphs(qg_model *m)
 {
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < 4; i++) {
         if (m->g_fwd[i]) (void)hipGraphExecDestroy(m->g_fwd[i]);
         if (m->g_dec[i]) (void)hipGraphExecDestroy(m->g_dec[i]);
         m->g_fwd[i] = m->g_dec[i] = nullptr;
@@ -1208,22 +1405,32 @@ int enqueue_forward(qg_model *m)
                     hipLaunchKernelGGL(qgm::attn_rope_head_k<4>, grid, block, 0, st, aa, m->ao);
             } else {
                 const dim3 grid(c.n_heads / m->att_grp * m->att_nsplit);
-                if (m->hd == 64)
+                const bool vec = m->att_mode == 3;
+                if (vec && m->hd == 128)
+                    hipLaunchKernelGGL(qgm::attn_rope_split_vec_k<2>, grid, dim3(256), 0, st, aa);
+                else if (vec)                                    // head_dim 256 (vec_seq)
+                    hipLaunchKernelGGL(qgm::attn_rope_split_vec_k<4>, grid, dim3(256), 0, st, aa);
+                else if (m->hd == 64)
                     hipLaunchKernelGGL(qgm::attn_rope_split_k<1>, grid, dim3(256), 0, st, aa);
                 else if (m->hd == 128)
                     hipLaunchKernelGGL(qgm::attn_rope_split_k<2>, grid, dim3(256), 0, st, aa);
                 else
                     hipLaunchKernelGGL(qgm::attn_rope_split_k<4>, grid, dim3(256), 0, st, aa);
-                const dim3 cg(c.n_heads), cb(1024);
-                if (m->hd == 64)
-                    hipLaunchKernelGGL(qgm::attn_combine_k<1>, cg, cb, 0, st, m->att_part, m->att_ml, m->ao, m->d_step,
-                                       m->att_nsplit);
+                const bool few = m->att_nsplit <= qgm::kFewSplit;
+                auto combine = [&](auto kernel) {
+                    hipLaunchKernelGGL(kernel, dim3(c.n_heads), dim3(few ? 256 : 1024), 0, st, m->att_part, m->att_ml,
+                                       m->ao, m->d_step, m->att_nsplit);
+                };
+                if (vec && m->hd == 128)
+                    combine(few ? qgm::attn_combine_k<2, 4, true> : qgm::attn_combine_k<2, 16, true>);
+                else if (vec)
+                    combine(few ? qgm::attn_combine_k<4, 4, true> : qgm::attn_combine_k<4, 16, true>);
+                else if (m->hd == 64)
+                    combine(few ? qgm::attn_combine_k<1, 4, false> : qgm::attn_combine_k<1, 16, false>);
                 else if (m->hd == 128)
-                    hipLaunchKernelGGL(qgm::attn_combine_k<2>, cg, cb, 0, st, m->att_part, m->att_ml, m->ao, m->d_step,
-                                       m->att_nsplit);
+                    combine(few ? qgm::attn_combine_k<2, 4, false> : qgm::attn_combine_k<2, 16, false>);
                 else
-                    hipLaunchKernelGGL(qgm::attn_combine_k<4>, cg, cb, 0, st, m->att_part, m->att_ml, m->ao, m->d_step,
-                                       m->att_nsplit);
+                    combine(few ? qgm::attn_combine_k<4, 4, false> : qgm::attn_combine_k<4, 16, false>);
             }
         } else {
             hipLaunchKernelGGL(qgm::qkv_post_k, dim3((pairs + 255) / 256), dim3(256), 0, st, m->q, m->k, m->v,
@@ -1329,15 +1536,17 @@ bool two_range_ok(const qg_model *m)
 // the attention mode of the forward pass that writes cache slot `slot`: up to
 // kShortSeq cached positions whole heads as two position ranges per head
 // where every wo takes them (mode 2), else up to short_seq1 in one workgroup
-// per head (mode 1); beyond, split over position ranges (mode 0).  att_path: 0 by length, 1
-// always one workgroup per head, 2 always split, 3 always two ranges where
-// the wo matrices allow it (else one workgroup per head).
+// per head (mode 1); beyond, split over position ranges (mode 3 up to vec_seq,
+// then mode 0).  att_path: 0 by length, 1 always one workgroup per head, 2
+// always split, 3 always two ranges where the wo matrices allow it (else one
+// workgroup per head).
 void pick_attention(qg_model *m, uint32_t slot)
 {
     const int whole = m->att_path != 1 && two_range_ok(m) ? 2 : 1;
     const uint32_t most = whole == 2 ? qgm::kShortSeq : qgm::short_seq1(m->hd);
     const bool shrt = m->att_path == 1 || m->att_path == 3 || (m->att_path == 0 && slot + 1 <= most);
-    m->att_mode = m->att_grp && shrt ? whole : 0;
+    const int split = m->att_grp && slot + 1 <= qgm::vec_seq(m->hd, m->att_grp) ? 3 : 0;
+    m->att_mode = m->att_grp && shrt ? whole : split;
 }
 
 int run_forward(qg_model *m, uint32_t slot)

@@ -1,5 +1,5 @@
-"""The split decode attention (attn_rope_split_k, attn_combine_k) against the
-oracle where its tiles and ranges end: 1 to 65 cached positions (a wave of 16
+"""The split decode attention (attn_rope_split_k and attn_rope_split_vec_k,
+attn_combine_k) against the oracle where its tiles and ranges end: 1 to 65 cached positions (a wave of 16
 with none, one and all of its positions, the second tile of 64), 4100 (ranges
 of two tiles), grouped heads of every size up to 8 and one, head_dim 64, 128
 and 256.  The prompt goes through the token-by-token path up to 70 positions,
@@ -15,7 +15,8 @@ from test_decode_gpu import SMALL, build
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("embed,heads,kv", [(256, 4, 2), (448, 7, 1), (512, 8, 1), (1024, 8, 8), (1024, 4, 1)])
+@pytest.mark.parametrize("embed,heads,kv", [(256, 4, 2), (448, 7, 1), (512, 8, 1), (512, 4, 2), (1024, 8, 1), (1024, 8, 8),
+                                            (1024, 4, 1), (2048, 16, 16), (4096, 16, 16)])
 def test_every_length(rinf, synth, oracle, ctx, embed, heads, kv):
     cfg = dict(SMALL, embed_dim=embed, n_heads=heads, n_kv_heads=kv, n_layers=1)
     dev, ref, _ = build(rinf, synth, oracle, ctx, cfg, "q8_0", 31, 80)
@@ -87,6 +88,24 @@ def test_ranges_of_many_groups(rinf, synth, oracle, ctx):
         ref.forward(int(tok), pos)
     logits = np.zeros(300, np.float32)
     for i in range(30):
+        dev.forward(i, n + i, logits)
+        assert normwise_err(logits, ref.forward(i, n + i)) <= TIGHT_TOL, i
+    dev.close()
+
+
+@pytest.mark.parametrize("embed,heads,kv,most", [(1280, 5, 1, 1280), (256, 2, 2, 832), (1024, 4, 1, 2560)])
+def test_where_the_vector_units_end(rinf, synth, oracle, ctx, embed, heads, kv, most):
+    """Across the length at which attn_rope_split_vec_k (head_dim 256, and 128 with a
+    kv head per head) gives way to attn_rope_split_k."""
+    cfg = dict(SMALL, embed_dim=embed, n_heads=heads, n_kv_heads=kv, hidden_dim=256, n_layers=1, vocab_size=300)
+    n = most - 8
+    dev, ref, _ = build(rinf, synth, oracle, ctx, cfg, "q8_0", 36, n + 20)
+    prompt = np.random.default_rng(7).integers(0, 300, n)
+    dev.prefill(prompt)
+    for pos, tok in enumerate(prompt):
+        ref.forward(int(tok), pos)
+    logits = np.zeros(300, np.float32)
+    for i in range(20):
         dev.forward(i, n + i, logits)
         assert normwise_err(logits, ref.forward(i, n + i)) <= TIGHT_TOL, i
     dev.close()
