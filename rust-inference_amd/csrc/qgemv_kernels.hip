@@ -432,6 +432,7 @@ __device__ __forceinline__ float wave_sum(float v)
 // (K-quants: ~13 instructions per element, the header unpacked per quad).
 // Against one element per lane at a time: F16 3001 x 2050 12.2 -> 4.4 us, Q4_K
 // 4096 x 14336 in the f32 mode 147 -> 34 us.
+constexpr uint32_t kQuadCols = 0xFFFFFFFFu - 1024u;              // a step of 256 threads past them does not wrap
 struct QuadArgs {
     const uint8_t *w;
     const float *x;
@@ -460,10 +461,9 @@ __global__ void __launch_bounds__(256) gemv_quads(QuadArgs a)
         acc[i] = 0.f;
     }
     auto add = [](float s, float p, float q) { return FUSE ? __builtin_fmaf(p, q, s) : s + p * q; };
-    if constexpr (AL) {                                          // cols % 4 == 0: rows start on quads
+    if constexpr (AL) {                                          // cols % 4 == 0: rows start on quads; cols <= kQuadCols
 #pragma unroll 4
-        for (uint32_t q = tid; q < a.cols / 4u; q += TPR) {      // (a counter of elements could wrap)
-            const uint32_t c = 4u * q;
+        for (uint32_t c = 4u * tid; c < a.cols; c += 4u * TPR) {
             const f4 x = *(const f4u *)(a.x + c);
 #pragma unroll
             for (uint32_t i = 0; i < R; i++) {
@@ -3216,11 +3216,13 @@ int launch_gemv_norm_pair(uint32_t t1, const Plan &p1, const uint8_t *w1, size_t
 
 // Long aligned rows share x between four rows of a workgroup where that
 // leaves four waves per SIMD (a row of 4 KB of x is one pass of its 256
-// threads); otherwise a wave per row.
+// threads); otherwise a wave per row.  Aligned rows count their elements (in
+// quads, as the others, f32 Q5_0 105 x 16128 took 10.5 us instead of 10.0), so
+// the longest go with the others.
 template <uint32_t T, bool RP, bool FUSE>
 static int launch_quads_t(const QuadArgs &a, hipStream_t st)
 {
-    const bool al = a.cols % 4u == 0;
+    const bool al = a.cols % 4u == 0 && a.cols <= kQuadCols;
     if (al && a.cols >= 4096u && a.rows >= 4096u)
         hipLaunchKernelGGL((gemv_quads<T, RP, FUSE, 256, 4, true>), dim3((a.rows + 3u) / 4u), dim3(256), 0, st, a);
     else if (al)
